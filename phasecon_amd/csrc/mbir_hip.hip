@@ -544,16 +544,18 @@ struct SweepLds {
 // Register staging of a column's A window and t+-1 values (prefetch): PI
 // first bins and PA values per lane (kSmall: frames of at most 64 views and
 // 256 window values).  kHalf: the values stay FP16 bits until they are
-// stored, so that no conversion waits on the loads in flight.
-template <bool kSmall, bool kHalf = false>
+// stored, so that no conversion waits on the loads in flight.  kNS
+// wavefronts share the staging, `me` the thread's index among them.
+template <bool kSmall, bool kHalf = false, int kNS = 1>
 struct APre {
-  static constexpr int PI = kSmall ? 1 : kPreI;
-  static constexpr int PA = kSmall ? 4 : kPreA;
+  static constexpr int PI = kSmall ? 1 : kPreI / kNS;
+  static constexpr int PA = kSmall ? 4 : kPreA / kNS;
+  static constexpr int PT = (kTnPre + kNS - 1) / kNS;
   using AV = typename std::conditional<kHalf, unsigned short, float>::type;
   int a0[PI];
   AV av[PA];
   float scale;
-  float tn[kTnPre];
+  float tn[PT];
 };
 
 // Window buffer b of the sweep's LDS by address arithmetic (the buffers are
@@ -568,20 +570,20 @@ __device__ __forceinline__ Win pick_win(const L_& L, int b) {
 
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (kWave - 1); }
 
-template <int kW, bool kSmall, bool kHalf = false>
+template <int kW, bool kSmall, bool kHalf = false, int kNS = 1>
 __device__ __forceinline__ void awin_fetch(const SwGeom& G, const ColumnArgs& A, int c, int s0,
-                                           int nv, APre<kSmall, kHalf>& pre) {
-  const int lane = lane_id();
+                                           int nv, int me, APre<kSmall, kHalf, kNS>& pre) {
+  using Pre = APre<kSmall, kHalf, kNS>;
   const size_t base = (size_t)c * G.nslots + s0;
 #pragma unroll
-  for (int i = 0; i < APre<kSmall, kHalf>::PI; ++i) {
-    const int j = lane + i * kWave;
+  for (int i = 0; i < Pre::PI; ++i) {
+    const int j = me + i * (kNS * kWave);
     pre.a0[i] = j < nv ? A.afirst[base + j] : -1;
   }
   const int nav = nv * kW;
 #pragma unroll
-  for (int i = 0; i < APre<kSmall, kHalf>::PA; ++i) {
-    const int j = lane + i * kWave;
+  for (int i = 0; i < Pre::PA; ++i) {
+    const int j = me + i * (kNS * kWave);
     if constexpr (kHalf)
       pre.av[i] = j < nav ? A.aval16[base * kW + j] : (unsigned short)0;
     else
@@ -591,12 +593,12 @@ __device__ __forceinline__ void awin_fetch(const SwGeom& G, const ColumnArgs& A,
 }
 
 // The t-1 and t+1 columns of voxel column c (not updated in a sweep launch).
-template <typename Pre>
+template <bool kSmall, bool kHalf, int kNS>
 __device__ __forceinline__ void tn_fetch(const SwGeom& G, const float* x, int f, int c,
-                                         size_t vol, Pre& pre) {
+                                         size_t vol, int me, APre<kSmall, kHalf, kNS>& pre) {
 #pragma unroll
-  for (int i = 0; i < kTnPre; ++i) {
-    const int j = lane_id() + i * kWave;
+  for (int i = 0; i < APre<kSmall, kHalf, kNS>::PT; ++i) {
+    const int j = me + i * (kNS * kWave);
     const int ff = j < G.N_z ? f - 1 : f + 1;
     const bool ok = j < 2 * G.N_z && ff >= 0 && ff < G.N_time;
     pre.tn[i] = ok ? x[(size_t)ff * vol + (size_t)c * G.N_z + j % G.N_z] : 0.f;
@@ -605,19 +607,20 @@ __device__ __forceinline__ void tn_fetch(const SwGeom& G, const float* x, int f,
 
 // Stores a prefetched window (first bins turned into sinogram offsets
 // through the frame's view list) and t+-1 values.
-template <int kW, bool kSmall, bool kHalf = false>
-__device__ __forceinline__ void awin_store(const SwGeom& G, const APre<kSmall, kHalf>& pre,
-                                           int nv, const int* views, const Win& win, float* tn) {
-  const int lane = lane_id();
+template <int kW, bool kSmall, bool kHalf = false, int kNS = 1>
+__device__ __forceinline__ void awin_store(const SwGeom& G,
+                                           const APre<kSmall, kHalf, kNS>& pre, int nv,
+                                           const int* views, int me, const Win& win, float* tn) {
+  using Pre = APre<kSmall, kHalf, kNS>;
 #pragma unroll
-  for (int i = 0; i < APre<kSmall, kHalf>::PI; ++i) {
-    const int j = lane + i * kWave;
+  for (int i = 0; i < Pre::PI; ++i) {
+    const int j = me + i * (kNS * kWave);
     if (j < nv) win.base[j] = pre.a0[i] >= 0 ? (views[j] * G.N_r + pre.a0[i]) * G.N_t : -1;
   }
   const int nav = nv * kW;
 #pragma unroll
-  for (int i = 0; i < APre<kSmall, kHalf>::PA; ++i) {
-    const int j = lane + i * kWave;
+  for (int i = 0; i < Pre::PA; ++i) {
+    const int j = me + i * (kNS * kWave);
     if constexpr (kHalf) {
       // the same product k_aquant wrote into the FP32 copy of A
       if (j < nav) win.av[j] = (float)__builtin_bit_cast(_Float16, pre.av[i]) * pre.scale;
@@ -626,8 +629,8 @@ __device__ __forceinline__ void awin_store(const SwGeom& G, const APre<kSmall, k
     }
   }
 #pragma unroll
-  for (int i = 0; i < kTnPre; ++i) {
-    const int j = lane + i * kWave;
+  for (int i = 0; i < Pre::PT; ++i) {
+    const int j = me + i * (kNS * kWave);
     if (j < 2 * G.N_z) tn[j] = pre.tn[i];
   }
 }
@@ -635,89 +638,75 @@ __device__ __forceinline__ void awin_store(const SwGeom& G, const APre<kSmall, k
 // Lane layout over a column's sinogram footprint: lane = (detector row rr,
 // slot group g), g fastest; a lane takes view slots g, g + groups, ... in row
 // rr (and rr + rpl, ... when N_t > 64).  A slot's W bins lie N_t apart in e
-// and w.  With a power-of-two rpl the slot groups of a row are `groups`
-// consecutive lanes, summed with DPP.
+// and w.  groups is a power of two (the most that fit beside rpl rows), so
+// that a row's groups are aligned consecutive lanes, summed with DPP.
 struct Lanes {
   int rpl, groups, g, rr;
-  bool pow2;
   __device__ Lanes(int N_t) {
     const int lane = lane_id();
     rpl = N_t < kWave ? N_t : kWave;
-    groups = kWave / rpl;
+    groups = 1 << (31 - __builtin_clz((unsigned)(kWave / rpl)));
     rr = lane / groups;
-    g = lane % groups;
-    pow2 = (rpl & (rpl - 1)) == 0;
+    g = lane & (groups - 1);
   }
 };
 
 // theta1/theta2 per detector row of one voxel column (XT_VoxUpdate.c:56-85,
-// generalized-Huber weight included).  Each lane issues the e/w loads of a
-// batch of its slots back to back, then accumulates; row sums land in
-// row1/row2 (part1/part2: LDS partials for the non-power-of-two case).
+// generalized-Huber weight included) by nw wavefronts, wavefront wv taking
+// the view slots (j nw + wv) groups + g, j = 0, 1, ...: its share of every
+// row's sums lands in row1 / row2.  Each lane issues the e/w loads of a batch
+// of its slots back to back, then accumulates; entries with a = 0 load an
+// address of their own batch's first element and are not used, so that no
+// branch splits the batch.
 template <int kW>
 __device__ __forceinline__ void col_thetas(const SwGeom& G, const ColumnArgs& A, const Win& win,
-                                           int nv, float* row1, float* row2, float* part1,
-                                           float* part2) {
-  constexpr int SB = kW <= 5 ? 2 : 1;  // slots per load batch
-  const int lane = lane_id();
+                                           int nv, int wv, int nw, float* row1, float* row2) {
+  constexpr int SB = kW <= 5 ? 4 : (kW <= 9 ? 2 : 1);  // slots per load batch
   const Lanes L(G.N_t);
+  const int step = nw * L.groups;
   const float T2 = G.huber_T * G.huber_T, Thd = G.huber_T * G.huber_delta;
   for (int t0 = 0; t0 < G.N_t; t0 += L.rpl) {
     const int row = t0 + L.rr;
     const bool lane_ok = L.rr < L.rpl && row < G.N_t;
     float a1 = 0.f, a2 = 0.f;
-    for (int sb = 0; sb < nv; sb += SB * L.groups) {
-      float ev[SB][kW], wv[SB][kW], av[SB][kW];
+    for (int sb = wv * L.groups; sb < nv; sb += SB * step) {
+      float el[SB][kW], wl[SB][kW];
 #pragma unroll
       for (int b = 0; b < SB; ++b) {
-        const int sl = sb + L.g + b * L.groups;
+        const int sl = sb + L.g + b * step;
         const int base = (lane_ok && sl < nv) ? win.base[sl] : -1;
 #pragma unroll
         for (int k = 0; k < kW; ++k) {
           const float a = base >= 0 ? win.av[sl * kW + k] : 0.f;
-          const bool ok = a != 0.f;
-          const int o = ok ? base + k * G.N_t + row : 0;
-          const float e = e_load(A.e + o);
-          ev[b][k] = ok ? e : 0.f;
-          wv[b][k] = ok ? A.w[o] : 0.f;
-          av[b][k] = a * G.delta_t;
+          const int o = a != 0.f ? base + k * G.N_t + row : 0;
+          el[b][k] = e_load(A.e + o);
+          wl[b][k] = A.w[o];
         }
       }
 #pragma unroll
-      for (int b = 0; b < SB; ++b)
+      for (int b = 0; b < SB; ++b) {
+        const int sl = sb + L.g + b * step;
+        const int base = (lane_ok && sl < nv) ? win.base[sl] : -1;
 #pragma unroll
         for (int k = 0; k < kW; ++k) {
+          const float av = base >= 0 ? win.av[sl * kW + k] : 0.f;
           // |e sqrt(w)| < T tested as e^2 w < T^2; the generalized-Huber
           // weight T delta sqrt(w)/|e| only where an entry is an outlier
-          const float e = ev[b][k], w = wv[b][k], a = av[b][k];
+          const float e = av != 0.f ? el[b][k] : 0.f, w = av != 0.f ? wl[b][k] : 0.f;
+          const float a = av * G.delta_t;
           float hw = w;
           if (e * e * w >= T2) hw = Thd * sqrtf(w) * __builtin_amdgcn_rcpf(fabsf(e));
           a2 += a * a * hw;
           a1 -= e * a * hw;
         }
-    }
-    if (L.pow2) {
-      a1 = group_sum(a1, L.groups);
-      a2 = group_sum(a2, L.groups);
-      if (L.g == 0 && row < G.N_t) {
-        row1[row] = a1;
-        row2[row] = a2;
-      }
-    } else {
-      part1[lane] = a1;
-      part2[lane] = a2;
-      wave_sync();
-      if (lane < L.rpl && t0 + lane < G.N_t) {
-        float s1 = 0.f, s2 = 0.f;
-        for (int gg = 0; gg < L.groups; ++gg) {
-          s1 += part1[lane * L.groups + gg];
-          s2 += part2[lane * L.groups + gg];
-        }
-        row1[t0 + lane] = s1;
-        row2[t0 + lane] = s2;
       }
     }
-    wave_sync();
+    a1 = group_sum(a1, L.groups);
+    a2 = group_sum(a2, L.groups);
+    if (L.g == 0 && lane_ok) {
+      row1[row] = a1;
+      row2[row] = a2;
+    }
   }
 }
 
@@ -803,17 +792,18 @@ __device__ __forceinline__ void theta_finish(const SwGeom& G, const Win& win, co
 }
 
 // e -= A delta_t dx along one voxel column (XT_VoxUpdate.c:96-116), with
-// atomics because other wavefronts' columns share detector bins.
+// atomics because other wavefronts' columns share detector bins; wavefront wv
+// of nw takes the view slots it takes in col_thetas.
 template <int kW>
 __device__ __forceinline__ void col_update(const SwGeom& G, const ColumnArgs& A, const Win& win,
-                                           int nv, const float* dxz) {
+                                           int nv, const float* dxz, int wv = 0, int nw = 1) {
   const Lanes L(G.N_t);
   for (int t0 = 0; t0 < G.N_t; t0 += L.rpl) {
     const int row = t0 + L.rr;
     if (L.rr >= L.rpl || row >= G.N_t) continue;
     const float dz = dxz[row / G.zo];
     if (dz == 0.f) continue;
-    for (int sl = L.g; sl < nv; sl += L.groups) {
+    for (int sl = wv * L.groups + L.g; sl < nv; sl += nw * L.groups) {
       const int base = win.base[sl];
       if (base < 0) continue;
 #pragma unroll
@@ -1007,7 +997,8 @@ struct SolveStats {
 // fixed part plus the column's own z-1 / z+1 neighbours at their current
 // values, zero skipping (XT_VoxUpdate.c:238-262), the surrogate minimiser and
 // over-relaxation (XT_ICD_update.c:174-176).  New values go to the slab,
-// changes to dxz.
+// changes to dxz.  row1 / row2: kNS shares of the rows' theta sums.
+template <int kNS>
 __device__ __forceinline__ void col_solve(const SwGeom& G, const PriorReg& R, float* sx,
                                           int centre0, int par, int iter, float alpha,
                                           const float* fnum, const float* fden,
@@ -1040,10 +1031,12 @@ __device__ __forceinline__ void col_solve(const SwGeom& G, const PriorReg& R, fl
   float xn = V;
   if (!skip) {
     float th1 = 0.f, th2 = 0.f;
-    for (int m = 0; m < G.zo; ++m) {
-      th1 += row1[z * G.zo + m];
-      th2 += row2[z * G.zo + m];
-    }
+    for (int m = 0; m < G.zo; ++m)
+#pragma unroll
+      for (int q = 0; q < kNS; ++q) {
+        th1 += row1[q * kNTMax + z * G.zo + m];
+        th2 += row2[q * kNTMax + z * G.zo + m];
+      }
     xn = substitute(alpha, V, th1, th2, num, den);
   }
   sx[centre] = xn;
@@ -1094,47 +1087,58 @@ struct SweepArgs {
   unsigned* xcd_check;  // [0] items run, [1] items off their XCD (may be null)
 };
 
-constexpr int kSweepThreads = 2 * kWave;
 constexpr int kXcds = 8;          // XCDs of an MI355X, each with its own L2
 constexpr int kHwRegXccId = 20;   // s_getreg id of XCC_ID (gfx940 family)
-constexpr int kNhMax = 2 * kSweepThreads;  // tile columns a non-homogeneous pass can rank
+constexpr int kNhMax = 256;       // tile columns a non-homogeneous pass can rank
 
 // One ICD pass over the voxel columns of the tiles in this launch (one
-// 2x2-checkerboard colour) for the frames of one parity, one workgroup of two
-// wavefronts per (tile, frame).  The tile's object slab plus a one-column
-// halo lives in LDS for the whole pass (neighbouring tiles and adjacent frames
-// are not updated in the same launch, so the halo and the t+-1 values are
-// constant), with the tile's column list and the frame's view list.  Per
-// column, in two barrier-separated phases:
-//   1. wavefront 0 computes theta1/theta2 from the shared error sinogram and
-//      prefetches the next column's A window and t+-1 values into registers,
-//      while wavefront 1 evaluates the surrogate's terms of the neighbours
-//      outside the column;
-//   2. wavefront 1 solves the z-parity halves (each voxel sees its z+-1
-//      neighbours' new values) while wavefront 0 stores the prefetch;
-// then wavefront 0 sends the column's error update with atomics and moves on
-// to the next column's theta while wavefront 1 starts its terms.
+// 2x2-checkerboard colour) for the frames of one parity, one workgroup per
+// (tile, frame): kNS wavefronts on the sinogram side and one on the prior
+// side.  The tile's object slab plus a one-column halo lives in LDS for the
+// whole pass (neighbouring tiles and adjacent frames are not updated in the
+// same launch, so the halo and the t+-1 values are constant), with the tile's
+// column list and the frame's view list.  Per column, in two
+// barrier-separated phases:
+//   1. the sinogram side computes theta1/theta2 from the shared error
+//      sinogram while the prior wavefront evaluates the surrogate's terms of
+//      the neighbours outside the column;
+//   2. the prior wavefront solves the z-parity halves (each voxel sees its
+//      z+-1 neighbours' new values).
+// kNS = 1, where a column's whole window is one load batch of one wavefront
+// (sweep_pipes): theta is pipelined -- the next column's loads go out during
+// the solve, and are corrected for the column's own update, whose atomics
+// follow.  kNS = 2 or 4 elsewhere: the view slots are dealt over kNS
+// wavefronts, so that a column is still one load batch per lane (one memory
+// round trip) and not a chain of them; each wavefront sends the error update
+// of its own slots and then loads them for the next column, so a column sees
+// its own tile's updates without a correction.  Bound by that chain (update,
+// load, sum, solve), not by bandwidth: 150 columns x 24 rows at half
+// resolution, 29 views per frame, W = 5, tile 8: 1.191 -> 0.418 ms per launch (6.5 us per column).
 // kW = W, the A window width.
-// The small-frame variants with window widths up to 5 are held to 128 VGPRs
-// (four wavefronts per SIMD, two spilled registers at W = 5): at 128x128x4
-// with tile 4 a launch's 2048 workgroups then fit the chip at once instead
-// of in two rounds.
-template <int kW, bool kSmall, bool kHalf>
-__global__ __launch_bounds__(kSweepThreads)
-__attribute__((amdgpu_waves_per_eu((kSmall && kW <= 5) ? 4 : 1))) void k_sweep(SwGeom G,
-                                                                              SweepArgs A) {
+// The small-frame pipelined variants with window widths up to 5 are compiled
+// for exactly four wavefronts per SIMD: at 128x128x4 with tile 4 a launch's
+// 2048 workgroups then fit the chip at once instead of in two rounds, and the
+// scheduler, free to use 128 VGPRs, keeps the pipelined loads in flight (left
+// to aim for five it takes 88 VGPRs and 0.672 instead of 0.600 ms per launch
+// at 256x256x8, tile 8, paired).
+template <int kW, bool kSmall, bool kHalf, int kNS>
+__global__ __launch_bounds__((kNS + 1) * kWave)
+__attribute__((amdgpu_waves_per_eu((kSmall && kW <= 5 && kNS == 1) ? 4 : 1,
+                                   (kSmall && kW <= 5 && kNS == 1) ? 4 : 8))) void
+k_sweep(SwGeom G, SweepArgs A) {
+  constexpr int kThreads = (kNS + 1) * kWave;
   extern __shared__ __align__(16) float smem[];
   __shared__ float s_tn[kWinBufs][2 * kNZMax];
-  __shared__ float s_row1[kNTMax], s_row2[kNTMax];
-  __shared__ float s_part1[kWave], s_part2[kWave];
+  __shared__ float s_row1[kNS * kNTMax], s_row2[kNS * kNTMax];
   __shared__ float s_dx[kNZMax], s_fnum[kNZMax], s_fden[kNZMax];
   __shared__ int s_fpos[kNZMax];
   __shared__ PriorTab s_prior;
   const int tid = threadIdx.x;
-  // wavefront 0: sinogram side; 1: prior side.  Read from lane 0 into a
-  // scalar register, so the role branch is a uniform (scalar) branch and each
-  // wavefront executes only its own loop's barriers.
-  const bool w0 = __builtin_amdgcn_readfirstlane(tid) < kWave;
+  // wavefronts 0 .. kNS-1: sinogram side; kNS: prior side.  Read from lane 0
+  // into a scalar register, so the role branch is a uniform (scalar) branch
+  // and each wavefront executes only its own loop's barriers.
+  const int wv = kNS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid) / kWave;
+  const bool w0 = __builtin_amdgcn_readfirstlane(tid) < kNS * kWave;
   const int wid_all = blockIdx.x;
   const int iter = A.iter_dev ? *A.iter_dev + A.iter : A.iter;
   load_prior(G, &s_prior);
@@ -1194,11 +1198,11 @@ __attribute__((amdgpu_waves_per_eu((kSmall && kW <= 5) ? 4 : 1))) void k_sweep(S
     pb = (int)(mix32(h + 0x9e3779b9u) % (unsigned)n);
   }
   // the tile's slab with halo (8 loads per thread in flight), column and view lists
-  for (int j0 = tid; j0 < nx; j0 += 8 * kSweepThreads) {
+  for (int j0 = tid; j0 < nx; j0 += 8 * kThreads) {
     float v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int j = j0 + u * kSweepThreads;
+      const int j = j0 + u * kThreads;
       const int z = j % Nz, b = j / Nz;
       const int yy = oy + b / BW, xx = ox + b % BW;
       v[u] = (j < nx && yy >= 0 && yy < G.N_y && xx >= 0 && xx < G.N_x)
@@ -1207,21 +1211,22 @@ __attribute__((amdgpu_waves_per_eu((kSmall && kW <= 5) ? 4 : 1))) void k_sweep(S
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u)
-      if (j0 + u * kSweepThreads < nx) L.x[j0 + u * kSweepThreads] = v[u];
+      if (j0 + u * kThreads < nx) L.x[j0 + u * kThreads] = v[u];
   }
-  for (int j = tid; j < n_all; j += kSweepThreads) L.cols[j] = A.tile_cols[c0 + j];
-  for (int j = tid; j < nv; j += kSweepThreads) L.views[j] = A.col.frame_views[s0 + j];
+  for (int j = tid; j < n_all; j += kThreads) L.cols[j] = A.tile_cols[c0 + j];
+  for (int j = tid; j < nv; j += kThreads) L.views[j] = A.col.frame_views[s0 + j];
   if (n < n_all) {
     // non-homogeneous pass: rank the tile's columns by nh_rank (the count of
     // columns ranked above, ties to the earlier entry, so the ranks are a
     // permutation) and compact the n highest to the front of the list
     const float* rk = A.nh_rank + (size_t)f * G.N_y * G.N_x;
-    for (int j = tid; j < n_all; j += kSweepThreads) s_row1[j] = rk[L.cols[j]];
+    for (int j = tid; j < n_all; j += kThreads) s_row1[j] = rk[L.cols[j]];
     __syncthreads();
-    int keep_c[kNhMax / kSweepThreads], keep_r[kNhMax / kSweepThreads];
+    constexpr int kKeep = (kNhMax + kThreads - 1) / kThreads;
+    int keep_c[kKeep], keep_r[kKeep];
 #pragma unroll
-    for (int u = 0; u < kNhMax / kSweepThreads; ++u) {
-      const int j = tid + u * kSweepThreads;
+    for (int u = 0; u < kKeep; ++u) {
+      const int j = tid + u * kThreads;
       keep_r[u] = n_all;
       keep_c[u] = 0;
       if (j < n_all) {
@@ -1237,23 +1242,18 @@ __attribute__((amdgpu_waves_per_eu((kSmall && kW <= 5) ? 4 : 1))) void k_sweep(S
     }
     __syncthreads();
 #pragma unroll
-    for (int u = 0; u < kNhMax / kSweepThreads; ++u)
+    for (int u = 0; u < kKeep; ++u)
       if (keep_r[u] < n) L.cols[keep_r[u]] = keep_c[u];
   }
   __syncthreads();
   int pos = pb;  // visiting order: pos_k = (pb + k pa) mod n
-  // the theta pipeline applies when a column's window is one load batch per
-  // lane (every slot of a lane's row in SB slots, N_t <= 64, a power of two)
-  constexpr int SB = ThetaLoads<kW>::SB;
-  const int rpl = G.N_t < kWave ? G.N_t : kWave;
-  const bool pipe = G.N_t <= kWave && (G.N_t & (G.N_t - 1)) == 0 && nv <= SB * (kWave / rpl);
   if (w0) {
     // window and t+-1 values of the first column
-    APre<kSmall, kHalf> pre;
+    APre<kSmall, kHalf, kNS> pre;
     const int cf = L.cols[pos];
-    awin_fetch<kW, kSmall, kHalf>(G, A.col, cf, s0, nv, pre);
-    tn_fetch(G, A.x, f, cf, vol, pre);
-    awin_store<kW, kSmall, kHalf>(G, pre, nv, L.views, L.win[0], s_tn[0]);
+    awin_fetch<kW, kSmall, kHalf, kNS>(G, A.col, cf, s0, nv, tid, pre);
+    tn_fetch(G, A.x, f, cf, vol, tid, pre);
+    awin_store<kW, kSmall, kHalf, kNS>(G, pre, nv, L.views, tid, L.win[0], s_tn[0]);
   }
   // nothing stays in flight: keeps the compiler's wait analysis from
   // carrying these loads into the column loop
@@ -1262,23 +1262,21 @@ __attribute__((amdgpu_waves_per_eu((kSmall && kW <= 5) ? 4 : 1))) void k_sweep(S
   SolveStats st;
   // Each wavefront runs its own loop over the columns; both loops pass the
   // same two workgroup barriers per column, so the phases stay aligned.
-  if (w0) {
+  if (w0 && kNS == 1) {
     const int lognt = __builtin_ctz((unsigned)G.N_t);
     ThetaLoads<kW> tl;
     // pipeline: the prefetch of column k+1 is in flight during column k's
     // solve, and stored at the start of column k's step (before the theta
     // loads of column k+1 go out)
-    APre<kSmall, kHalf> pre;
-    if (pipe) {
-      if (n > 1) {
-        int p1 = pos + pa;
-        if (p1 >= n) p1 -= n;
-        const int cn = L.cols[p1];
-        awin_fetch<kW, kSmall, kHalf>(G, A.col, cn, s0, nv, pre);
-        tn_fetch(G, A.x, f, cn, vol, pre);
-      }
-      theta_issue<kW>(G, A.col, L.win[0], nv, tl);
+    APre<kSmall, kHalf, kNS> pre;
+    if (n > 1) {
+      int p1 = pos + pa;
+      if (p1 >= n) p1 -= n;
+      const int cn = L.cols[p1];
+      awin_fetch<kW, kSmall, kHalf, kNS>(G, A.col, cn, s0, nv, tid, pre);
+      tn_fetch(G, A.x, f, cn, vol, tid, pre);
     }
+    theta_issue<kW>(G, A.col, L.win[0], nv, tl);
     for (int k = 0; k < n; ++k) {
       const int bc = k % kWinBufs, bn = (k + 1) % kWinBufs, bp = (k + 2) % kWinBufs;
       const Win wcur = pick_win(L, bc), wnext = pick_win(L, bn);
@@ -1288,43 +1286,51 @@ __attribute__((amdgpu_waves_per_eu((kSmall && kW <= 5) ? 4 : 1))) void k_sweep(S
       int p2 = p1 + pa;
       if (p2 >= n) p2 -= n;
       pos = p1;
-      if (pipe) {
-        // phase 1: theta of column k from the loads issued during the last
-        // solve, corrected for column k-1's own update; that update's
-        // atomics; column k+1's prefetch (it landed with the theta loads)
-        // stored over column k-2's window; the prefetch of column k+2
-        theta_finish<kW>(G, wcur, wprev, k > 0, s_dx, lognt, nv, tl, s_row1, s_row2);
-        if (k > 0) col_update<kW>(G, A.col, wprev, nv, s_dx);
-        if (k + 1 < n) awin_store<kW, kSmall, kHalf>(G, pre, nv, L.views, wnext, s_tn[bn]);
-        if (k + 2 < n) {
-          const int cn = L.cols[p2];
-          awin_fetch<kW, kSmall, kHalf>(G, A.col, cn, s0, nv, pre);
-          tn_fetch(G, A.x, f, cn, vol, pre);
-        }
-        __syncthreads();
-        // phase 2 (during the solve of column k): column k+1's theta loads
-        if (k + 1 < n) theta_issue<kW>(G, A.col, wnext, nv, tl);
-        __syncthreads();
-      } else {
-        // phase 1: prefetch of column k+1, theta of column k
-        if (k + 1 < n) {
-          const int cn = L.cols[p1];
-          awin_fetch<kW, kSmall, kHalf>(G, A.col, cn, s0, nv, pre);
-          tn_fetch(G, A.x, f, cn, vol, pre);
-        }
-        col_thetas<kW>(G, A.col, wcur, nv, s_row1, s_row2, s_part1, s_part2);
-        __syncthreads();
-        // phase 2: store the prefetch (it landed with the theta loads) and
-        // retire every load explicitly (a free wait here) so that the
-        // compiler's wait analysis carries none into the next column, before
-        // the error update's atomics go out
-        if (k + 1 < n) awin_store<kW, kSmall, kHalf>(G, pre, nv, L.views, wnext, s_tn[bn]);
-        __builtin_amdgcn_s_waitcnt(0);
-        __syncthreads();
-        col_update<kW>(G, A.col, wcur, nv, s_dx);
+      // phase 1: theta of column k from the loads issued during the last
+      // solve, corrected for column k-1's own update; that update's
+      // atomics; column k+1's prefetch (it landed with the theta loads)
+      // stored over column k-2's window; the prefetch of column k+2
+      theta_finish<kW>(G, wcur, wprev, k > 0, s_dx, lognt, nv, tl, s_row1, s_row2);
+      if (k > 0) col_update<kW>(G, A.col, wprev, nv, s_dx);
+      if (k + 1 < n)
+        awin_store<kW, kSmall, kHalf, kNS>(G, pre, nv, L.views, tid, wnext, s_tn[bn]);
+      if (k + 2 < n) {
+        const int cn = L.cols[p2];
+        awin_fetch<kW, kSmall, kHalf, kNS>(G, A.col, cn, s0, nv, tid, pre);
+        tn_fetch(G, A.x, f, cn, vol, tid, pre);
       }
+      __syncthreads();
+      // phase 2 (during the solve of column k): column k+1's theta loads
+      if (k + 1 < n) theta_issue<kW>(G, A.col, wnext, nv, tl);
+      __syncthreads();
     }
-    if (pipe) col_update<kW>(G, A.col, pick_win(L, (n - 1) % kWinBufs), nv, s_dx);
+    col_update<kW>(G, A.col, pick_win(L, (n - 1) % kWinBufs), nv, s_dx);
+  } else if (w0) {
+    APre<kSmall, kHalf, kNS> pre;
+    for (int k = 0; k < n; ++k) {
+      const int bn = (k + 1) % kWinBufs;
+      const Win wcur = pick_win(L, k % kWinBufs), wnext = pick_win(L, bn);
+      int p1 = pos + pa;
+      if (p1 >= n) p1 -= n;
+      pos = p1;
+      // phase 1: prefetch of column k+1, theta of column k
+      if (k + 1 < n) {
+        const int cn = L.cols[p1];
+        awin_fetch<kW, kSmall, kHalf, kNS>(G, A.col, cn, s0, nv, tid, pre);
+        tn_fetch(G, A.x, f, cn, vol, tid, pre);
+      }
+      col_thetas<kW>(G, A.col, wcur, nv, wv, kNS, s_row1 + wv * kNTMax, s_row2 + wv * kNTMax);
+      __syncthreads();
+      // phase 2: store the prefetch (it landed with the theta loads) and
+      // retire every load explicitly (a free wait here) so that the
+      // compiler's wait analysis carries none into the next column, before
+      // the error update's atomics go out
+      if (k + 1 < n)
+        awin_store<kW, kSmall, kHalf, kNS>(G, pre, nv, L.views, tid, wnext, s_tn[bn]);
+      __builtin_amdgcn_s_waitcnt(0);
+      __syncthreads();
+      col_update<kW>(G, A.col, wcur, nv, s_dx, wv, kNS);
+    }
   } else {
     PriorReg R;
     R.load(s_prior);
@@ -1346,10 +1352,10 @@ __attribute__((amdgpu_waves_per_eu((kSmall && kW <= 5) ? 4 : 1))) void k_sweep(S
         col_fixed(G, s_prior, L.x, BW, ly, lx, cy, cx, f, tcur, s_fnum, s_fden, s_fpos);
       __syncthreads();
       // phase 2: the z-parity halves
-      col_solve(G, R, L.x, centre0, 0, iter, A.alpha, s_fnum, s_fden, s_fpos, s_row1, s_row2,
+      col_solve<kNS>(G, R, L.x, centre0, 0, iter, A.alpha, s_fnum, s_fden, s_fpos, s_row1, s_row2,
                 s_dx, st);
       wave_sync();
-      col_solve(G, R, L.x, centre0, 1, iter, A.alpha, s_fnum, s_fden, s_fpos, s_row1, s_row2,
+      col_solve<kNS>(G, R, L.x, centre0, 1, iter, A.alpha, s_fnum, s_fden, s_fpos, s_row1, s_row2,
                 s_dx, st);
       __syncthreads();
       if (A.mag) {
@@ -1363,7 +1369,7 @@ __attribute__((amdgpu_waves_per_eu((kSmall && kW <= 5) ? 4 : 1))) void k_sweep(S
   }
   __syncthreads();
   // write the tile back (interior of the box, inside the object)
-  for (int j = tid; j < nx; j += kSweepThreads) {
+  for (int j = tid; j < nx; j += kThreads) {
     const int z = j % Nz, b = j / Nz;
     const int by = b / BW, bx = b % BW;
     if (by == 0 || bx == 0 || by == BW - 1 || bx == BW - 1) continue;
@@ -1377,7 +1383,7 @@ __attribute__((amdgpu_waves_per_eu((kSmall && kW <= 5) ? 4 : 1))) void k_sweep(S
       st.skip += __shfl_xor(st.skip, off);
       st.upd += __shfl_xor(st.upd, off);
     }
-    if (tid == kWave) {
+    if (lane_id() == 0) {
       atomicAdd(&A.stats[0], st.dx);
       atomicAdd(&A.stats[1], st.x);
       atomicAdd(&A.stats[2], st.skip);
@@ -1981,7 +1987,6 @@ __global__ __launch_bounds__(kWave) void k_thetas(SwGeom G, ColumnArgs A,
                                                   float* __restrict__ th2) {
   extern __shared__ __align__(16) float smem[];
   __shared__ float s_row1[kNTMax], s_row2[kNTMax];
-  __shared__ float s_part1[kWave], s_part2[kWave];
   __shared__ float s_tn[2 * kNZMax];
   const SweepLds L(smem, 0, nvmax, kW);
   const int i = blockIdx.x;
@@ -1991,12 +1996,13 @@ __global__ __launch_bounds__(kWave) void k_thetas(SwGeom G, ColumnArgs A,
   for (int j = threadIdx.x; j < nv; j += kWave) L.views[j] = A.frame_views[s0 + j];
   wave_sync();
   APre<false> pre;
-  awin_fetch<kW, false>(G, A, c, s0, nv, pre);
+  awin_fetch<kW, false>(G, A, c, s0, nv, lane_id(), pre);
   for (int q = 0; q < kTnPre; ++q) pre.tn[q] = 0.f;
-  awin_store<kW, false>(G, pre, nv, L.views, L.win[0], s_tn);
+  awin_store<kW, false>(G, pre, nv, L.views, lane_id(), L.win[0], s_tn);
   __builtin_amdgcn_s_waitcnt(0);
   wave_sync();
-  col_thetas<kW>(G, A, L.win[0], nv, s_row1, s_row2, s_part1, s_part2);
+  col_thetas<kW>(G, A, L.win[0], nv, 0, 1, s_row1, s_row2);
+  wave_sync();
   if (threadIdx.x == 0) {
     float a = 0.f, b = 0.f;
     for (int m = 0; m < G.zo; ++m) {
@@ -2634,6 +2640,16 @@ int run_fwdproj(mbir_hip_ctx* c, int mode, const float* x, float* out,
   return ev_end(c, mode == 1 ? MBIR_K_COST : MBIR_K_FWDPROJ);
 }
 
+template <int kW, bool kSmall, int kNS>
+void launch_sweep(mbir_hip_ctx* c, const SweepArgs& A, unsigned nwg, size_t lds) {
+  if (c->afp16)
+    hipLaunchKernelGGL((k_sweep<kW, kSmall, true, kNS>), dim3(nwg), dim3((kNS + 1) * kWave), lds,
+                       c->stream, c->SG, A);
+  else
+    hipLaunchKernelGGL((k_sweep<kW, kSmall, false, kNS>), dim3(nwg), dim3((kNS + 1) * kWave), lds,
+                       c->stream, c->SG, A);
+}
+
 int sum_partials(mbir_hip_ctx* c, size_t n, double* out) {
   std::vector<double> h(n);
   HIP_OK(hipMemcpyAsync(h.data(), c->d_partial, n * sizeof(double), hipMemcpyDeviceToHost,
@@ -3043,6 +3059,25 @@ int mbir_sweep_fits(const mbir_hip_ctx* c) {
   return 0;
 }
 
+// The pipelined sweep (one sinogram wavefront) runs where the largest frame's
+// window is one load batch of that wavefront: N_t a power of two up to 64 and
+// nvmax <= SB (64 / N_t) slots, SB = 2 up to W = 5, else 1.
+bool sweep_pipes(const mbir_hip_ctx* c) {
+  const int nt = c->g.N_t;
+  return nt <= kWave && (nt & (nt - 1)) == 0 &&
+         c->nvmax <= (c->G.W <= 5 ? 2 : 1) * (kWave / nt);
+}
+
+// Sinogram wavefronts of a launch of nwg workgroups: 4 where each gets a CU
+// of its own, so that a column is one short load batch; 2 in larger launches,
+// where the workgroups hide each other's latency and more of them at once
+// only crowd the error sinogram's atomics.  Measured (4 against 2, ms per
+// launch): 75 workgroups 0.418 / 0.704, 210 workgroups 0.310 / 0.326, 624
+// workgroups 0.660 / 0.412, 1712 workgroups 2.09 / 1.04.
+int sweep_waves(const mbir_hip_ctx* c, unsigned nwg) {
+  return sweep_pipes(c) ? 1 : (nwg <= 256 ? 4 : 2);
+}
+
 // The 8 launches per equit (2x2 tile colours x 2 frame parities) of n equits.
 // iter_dev null: iterations first_iter .. first_iter + n - 1, each launch
 // timed; otherwise the iteration is *iter_dev + it (graph capture: no event
@@ -3079,8 +3114,8 @@ int sweep_launches(mbir_hip_ctx* c, int32_t n, int32_t first_iter, uint32_t seed
     return fail("tile too large for N_z: the tile slab must fit 48 KiB of LDS");
   const size_t xbytes =
       sizeof(float) * sweep_lds_words(xfl, c->nvmax, c->G.W, c->tile * c->tile);
-  // static LDS of k_sweep (t+-1 buffers, row sums, per-voxel arrays) < 8 KiB
-  if (xbytes + 8 * 1024 > c->lds_max)
+  // static LDS of k_sweep (t+-1 buffers, row sums, per-voxel arrays) < 14 KiB
+  if (xbytes + (sweep_pipes(c) ? 8 : 14) * 1024 > c->lds_max)
     return fail("tile slab and A windows exceed the LDS of one workgroup");
   const int nf = c->g.N_time;
   const bool timed = iter_dev == nullptr;
@@ -3155,19 +3190,15 @@ int sweep_launches(mbir_hip_ctx* c, int32_t n, int32_t first_iter, uint32_t seed
           nwg += (unsigned)(set_ntl(b) * set_frames(b));
         }
         if (timed && ev_begin(c, MBIR_K_SWEEP)) return -1;
-        const dim3 grid(nwg), block(kSweepThreads);
-        if (small && c->afp16) {
-          MBIR_DISPATCH_W(c->G.W, hipLaunchKernelGGL((k_sweep<kW, true, true>), grid, block,
-                                                     xbytes, c->stream, c->SG, A));
-        } else if (small) {
-          MBIR_DISPATCH_W(c->G.W, hipLaunchKernelGGL((k_sweep<kW, true, false>), grid, block,
-                                                     xbytes, c->stream, c->SG, A));
-        } else if (c->afp16) {
-          MBIR_DISPATCH_W(c->G.W, hipLaunchKernelGGL((k_sweep<kW, false, true>), grid, block,
-                                                     xbytes, c->stream, c->SG, A));
+        const int ns = sweep_waves(c, nwg);
+        if (ns == 1 && small) {
+          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, true, 1>(c, A, nwg, xbytes)));
+        } else if (ns == 1) {
+          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, false, 1>(c, A, nwg, xbytes)));
+        } else if (ns == 2) {
+          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, false, 2>(c, A, nwg, xbytes)));
         } else {
-          MBIR_DISPATCH_W(c->G.W, hipLaunchKernelGGL((k_sweep<kW, false, false>), grid, block,
-                                                     xbytes, c->stream, c->SG, A));
+          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, false, 4>(c, A, nwg, xbytes)));
         }
         if (timed) {
           if (ev_end(c, MBIR_K_SWEEP)) return -1;

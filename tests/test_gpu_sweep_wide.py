@@ -1,0 +1,78 @@
+"""The sweep with its sinogram side on several wavefronts (windows that are
+not one load batch of one wavefront), voxel by voxel against the oracle's
+restatement of its schedule, as test_gpu_sweep_order.py does for the
+benchmark's shapes and with the same tolerance: one launch per tile colour
+and frame parity, so the sweep is the oracle's sequential ICD.
+
+The last test has launches of more workgroups than the chip has CUs, where
+the sinogram side takes two wavefronts and several tiles of a frame run at
+once: the maintained error sinogram stays y - A x and the cost falls.
+
+Shapes: row counts that are and are not powers of two and above one
+wavefront, view counts at both sides of a load batch and not a multiple of
+the slots that the wavefronts share.
+"""
+import numpy as np
+import pytest
+
+from test_gpu_sweep_order import TOL, _start
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,cols,views", [
+    (8, 32, 17), (8, 32, 33),     # just above one wavefront's load batch
+    (24, 32, 7), (24, 32, 29),    # 24 rows: 2 groups of 24 lanes
+    (12, 32, 20), (34, 16, 17),   # 4 groups of 12, one group of 34
+    (80, 16, 11)])                # rows above one wavefront
+def test_wide_sweep_matches_oracle_schedule(rows, cols, views):
+    from oracle.oracle import Oracle
+    from phasecon_amd.mbir import Stage
+    from phasecon_amd.synth import make_scan
+    scan = make_scan("tall3d", seed=1, rows=rows, cols=cols, views=views)
+    o = Oracle(scan)
+    T = cols // 2
+    print(f"rows {rows}, cols {cols}, views {views}", flush=True)
+    x0 = _start(o, 20, False)
+    st = Stage(scan, tile=T, alpha=1.5)
+    st.set_object(x0.astype(np.float32))
+    st.build_amatrix()
+    st.init_error()
+    st.icd(1, 21, 4242)
+    xg = st.get_object().astype(np.float64)
+    eg = st.get_error().astype(np.float64)
+    st.close()
+    xo = x0.copy()
+    eo = o.init_error(xo)
+    o.icd_equit_async(xo, eo, 21, T, 1.5, 4242, 0, 0, 0, 8, 0)
+    dx = np.abs(xg - xo).max() / np.abs(xo).max()
+    de = np.abs(eg - eo).max() / np.abs(o.y).max()
+    moved = np.abs(xo - x0).max() / np.abs(xo).max()
+    print(f"dx {dx:.3g} de {de:.3g} moved {moved:.3g}", flush=True)
+    assert moved > 100 * TOL
+    assert dx < TOL
+    assert de < TOL
+
+
+@pytest.mark.parametrize("rows,views", [(8, 20 * 16), (12, 7 * 16)])
+def test_wide_sweep_in_large_launches(rows, views):
+    from phasecon_amd.mbir import Stage
+    from phasecon_amd.synth import make_scan
+    scan = make_scan("ch4d_small", seed=2, rows=rows, views=views, frames=16)
+    print(f"rows {rows}, views {views}", flush=True)
+    st = Stage(scan, tile=4, alpha=1.0)   # about 50 tiles per colour x 8 frames
+    st.build_amatrix()
+    st.init_error()
+    costs = [st.cost()[0]]
+    for it in range(1, 7):
+        st.icd(1, it)
+        costs.append(st.cost()[0])
+    kept = st.get_error().astype(np.float64)
+    st.init_error()
+    fresh = st.get_error().astype(np.float64)
+    st.close()
+    d = np.abs(kept - fresh).max() / np.abs(st.y).max()
+    print(f"kept e off by {d:.3g}, costs {costs[0]:.6g} -> {costs[-1]:.6g}", flush=True)
+    # six equits of about 200 atomic additions per entry, each rounded to 2^-24
+    assert d < 2e-5
+    assert costs[-1] < 0.5 * costs[0]
