@@ -1085,6 +1085,12 @@ struct SweepArgs {
   // unit's items in unit_slots consecutive slots of that XCD
   int place_r, nfl, unit_slots;
   unsigned* xcd_check;  // [0] items run, [1] items off their XCD (may be null)
+  // the prior wavefront sends the error updates also for W >= 5 (always for
+  // W = 3): launches of at most a workgroup per CU, which are bound by the
+  // sinogram wavefront's chain (32x32x8, W = 5: 0.252 -> 0.231 ms); in full
+  // ones its 10 atomics per lane would delay the solve (128x128x4, 856
+  // workgroups: 0.241 -> 0.282 ms)
+  int prior_sends;
 };
 
 constexpr int kXcds = 8;          // XCDs of an MI355X, each with its own L2
@@ -1107,7 +1113,12 @@ constexpr int kNhMax = 256;       // tile columns a non-homogeneous pass can ran
 // kNS = 1, where a column's whole window is one load batch of one wavefront
 // (sweep_pipes): theta is pipelined -- the next column's loads go out during
 // the solve, and are corrected for the column's own update, whose atomics
-// follow.  kNS = 2 or 4 elsewhere: the view slots are dealt over kNS
+// follow.  The prior wavefront sends those after its fixed terms (it waits
+// for no load, so their completion is on nobody's path: the sinogram
+// wavefront's loads complete in order behind its own atomics) where W = 3 or
+// the launch is small (SweepArgs::prior_sends); measured against the
+// sinogram wavefront sending them, ms per launch: 32x32x4 0.206 -> 0.168,
+// 256x256x8 paired tile 8 0.599 -> 0.585, tile 12 0.617 -> 0.553.  kNS = 2 or 4 elsewhere: the view slots are dealt over kNS
 // wavefronts, so that a column is still one load batch per lane (one memory
 // round trip) and not a chain of them; each wavefront sends the error update
 // of its own slots and then loads them for the next column, so a column sees
@@ -1139,6 +1150,7 @@ k_sweep(SwGeom G, SweepArgs A) {
   // and each wavefront executes only its own loop's barriers.
   const int wv = kNS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid) / kWave;
   const bool w0 = __builtin_amdgcn_readfirstlane(tid) < kNS * kWave;
+  const bool prior_sends = kNS == 1 && (kW == 3 || A.prior_sends != 0);
   const int wid_all = blockIdx.x;
   const int iter = A.iter_dev ? *A.iter_dev + A.iter : A.iter;
   load_prior(G, &s_prior);
@@ -1287,11 +1299,12 @@ k_sweep(SwGeom G, SweepArgs A) {
       if (p2 >= n) p2 -= n;
       pos = p1;
       // phase 1: theta of column k from the loads issued during the last
-      // solve, corrected for column k-1's own update; that update's
-      // atomics; column k+1's prefetch (it landed with the theta loads)
-      // stored over column k-2's window; the prefetch of column k+2
+      // solve, corrected for column k-1's own update; that update's atomics
+      // (unless the prior side sends them); column k+1's prefetch (it landed
+      // with the theta loads) stored over column k-2's window; the prefetch
+      // of column k+2
       theta_finish<kW>(G, wcur, wprev, k > 0, s_dx, lognt, nv, tl, s_row1, s_row2);
-      if (k > 0) col_update<kW>(G, A.col, wprev, nv, s_dx);
+      if (k > 0 && !prior_sends) col_update<kW>(G, A.col, wprev, nv, s_dx);
       if (k + 1 < n)
         awin_store<kW, kSmall, kHalf, kNS>(G, pre, nv, L.views, tid, wnext, s_tn[bn]);
       if (k + 2 < n) {
@@ -1304,7 +1317,7 @@ k_sweep(SwGeom G, SweepArgs A) {
       if (k + 1 < n) theta_issue<kW>(G, A.col, wnext, nv, tl);
       __syncthreads();
     }
-    col_update<kW>(G, A.col, pick_win(L, (n - 1) % kWinBufs), nv, s_dx);
+    if (!prior_sends) col_update<kW>(G, A.col, pick_win(L, (n - 1) % kWinBufs), nv, s_dx);
   } else if (w0) {
     APre<kSmall, kHalf, kNS> pre;
     for (int k = 0; k < n; ++k) {
@@ -1350,6 +1363,8 @@ k_sweep(SwGeom G, SweepArgs A) {
         col_fixed_tab(G, R, NT, L.x, BW, ly, lx, cy, cx, tcur, s_fnum, s_fden, s_fpos);
       else
         col_fixed(G, s_prior, L.x, BW, ly, lx, cy, cx, f, tcur, s_fnum, s_fden, s_fpos);
+      if (prior_sends && k > 0)
+        col_update<kW>(G, A.col, pick_win(L, (k + 2) % kWinBufs), nv, s_dx);
       __syncthreads();
       // phase 2: the z-parity halves
       col_solve<kNS>(G, R, L.x, centre0, 0, iter, A.alpha, s_fnum, s_fden, s_fpos, s_row1, s_row2,
@@ -1366,6 +1381,7 @@ k_sweep(SwGeom G, SweepArgs A) {
         if (lane_id() == 0) A.mag[(size_t)f * G.N_y * G.N_x + c] = m;
       }
     }
+    if (prior_sends) col_update<kW>(G, A.col, pick_win(L, (n - 1) % kWinBufs), nv, s_dx);
   }
   __syncthreads();
   // write the tile back (interior of the box, inside the object)
@@ -3191,6 +3207,7 @@ int sweep_launches(mbir_hip_ctx* c, int32_t n, int32_t first_iter, uint32_t seed
         }
         if (timed && ev_begin(c, MBIR_K_SWEEP)) return -1;
         const int ns = sweep_waves(c, nwg);
+        A.prior_sends = nwg <= 256 ? 1 : 0;
         if (ns == 1 && small) {
           MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, true, 1>(c, A, nwg, xbytes)));
         } else if (ns == 1) {
