@@ -670,8 +670,9 @@ def calibration_copy(nbytes=1 << 30):
 def pcmbir_bench(views, n, sd_steps, nms, fft_reg=1):
     """Phase-retrieval throughput on one GPU at the PCMBIR workload's shape
     (views x n x n transforms, n = 512 the padded 256^2 detector): seconds
-    per steepest-descent iteration over all views (6 Fresnel transforms of
-    3 passes each per view), the FFT passes' HBM rate against 8 TB/s, and one
+    per steepest-descent iteration over all views (4 Fresnel transforms per
+    view in 5 row and 4 column passes that hold the elementwise steps; with
+    fft_reg 0 6 transforms of 3 passes each), the FFT passes' HBM rate against 8 TB/s, and one
     Nelder-Mead pass (pixels per second).  Synthetic data: a weak random phase
     object propagated by the same operator."""
     from phasecon_amd.pcmbir import PhaseRetrieval, wavelength, fresnel_window
@@ -696,9 +697,10 @@ def pcmbir_bench(views, n, sd_steps, nms, fft_reg=1):
     ctx.sd_run(sd_steps, 0.0)
     dt = (time.perf_counter() - t0) / sd_steps
     fft_ms, launches = ctx.fft_time()
-    per_transform_bytes = 3 * 2 * n * n * 8          # 3 passes, read + write, complex64
-    transforms = 6 * views * sd_steps                # 5 batched calls, one over 2 x views
-    gbps = per_transform_bytes * transforms / (fft_ms * 1e-3) / 1e9
+    # per pixel: the fused passes' 240 bytes (the first iteration's two more
+    # row passes left out), or 6 transforms of 3 passes, read + write, complex64
+    per_px = 240 if fft_reg else 6 * 3 * 2 * 8
+    gbps = per_px * views * n * n * sd_steps / (fft_ms * 1e-3) / 1e9
     out = {"pcmbir": {"views": views, "n": n, "fft": "register" if fft_reg else "lds-radix2",
                       "s_per_sd_iter": dt,
                       "fft_ms_per_sd_iter": fft_ms / sd_steps,

@@ -139,8 +139,9 @@ int pcmbir_hip_paganin(pcmbir_hip_ctx* ctx, const float* y, const float* D,
                        double delta_over_beta, double wavenumber, double* zr,
                        double* zi);
 
-/* Device time (ms) and launch count of the Fresnel FFT passes since the
- * last call, from HIP events on the context's stream. */
+/* Device time (ms) and launch count of the Fresnel FFT passes (with the
+ * steepest descent's elementwise steps and sums where they are fused into
+ * them) since the last call, from HIP events on the context's stream. */
 int pcmbir_hip_fft_time(pcmbir_hip_ctx* ctx, double* ms, int64_t* launches);
 
 #ifdef __cplusplus

@@ -15,10 +15,14 @@
 //                    factor (Fresnel phase, window, 1/N), inverse FFT along
 //                    rows, all in LDS -- one Fresnel transform is three passes
 //                    over the data (rows, columns, rows)
-//   k_pr_*           elementwise steps and per-view FP64 reductions of the
-//                    steepest descent (XT_PhaseRet.c), masked per view
+//   k_pr_rows        the steepest descent (XT_PhaseRet.c): inverse row FFT,
+//                    elementwise step, forward row FFT in one pass, with the
+//                    step's FP64 row sums, masked per view
+//   k_pr_*           its per-view sums; the elementwise steps on their own for
+//                    rows shorter than 8 values
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <cstring>
@@ -140,12 +144,14 @@ __host__ __device__ inline int col_tile(int logr, int logc) {
 }
 
 // Per (view, tile of TC columns): forward FFT along rows, times fac
-// [rows][cols], inverse FFT along rows.  LDS rows are padded by one value
+// [rows][cols], inverse FFT along rows (of the views whose active flag is
+// set; NULL: all).  LDS rows are padded by one value
 // against bank conflicts.
 __global__ __launch_bounds__(kThreads) void k_fresnel_cols(float2* __restrict__ data, int logr,
                                                            int logc,
                                                            const float2* __restrict__ twg,
-                                                           const float2* __restrict__ fac) {
+                                                           const float2* __restrict__ fac,
+                                                           const int* __restrict__ active) {
   __shared__ float2 s_buf[kColCap];
   __shared__ float2 s_tw[kFftMax / 2];
   const int rows = 1 << logr, cols = 1 << logc;
@@ -153,6 +159,7 @@ __global__ __launch_bounds__(kThreads) void k_fresnel_cols(float2* __restrict__ 
   const int stride = rows + 1;
   const int tiles = cols / TC;
   const int view = blockIdx.x / tiles, c0 = (blockIdx.x % tiles) * TC;
+  if (active && !active[view]) return;
   float2* base = data + ((size_t)view << (logr + logc)) + c0;
   for (int j = threadIdx.x; j < rows / 2; j += blockDim.x) s_tw[j] = twg[j];
   const int tot = rows * TC;
@@ -322,11 +329,20 @@ __host__ __device__ inline int col_tile_reg(int logr, int logc, int max_threads)
 __global__ __launch_bounds__(1024) void k_fresnel_cols_reg(float2* __restrict__ data, int logr,
                                                            int logc, int ltc,
                                                            const float2* __restrict__ twg,
-                                                           const float2* __restrict__ fac) {
+                                                           const float2* __restrict__ fac,
+                                                           const int* __restrict__ active) {
   extern __shared__ float2 s_ex[];
   const int TC = 1 << ltc, n8 = 1 << (logr - 3);
   const int tiles = 1 << (logc - ltc);
-  const int view = blockIdx.x >> (logc - ltc), c0 = (blockIdx.x & (tiles - 1)) << ltc;
+  // workgroups are dealt to the 8 XCDs round-robin: an XCD takes consecutive
+  // column tiles, so that the two halves of a 128-byte line are read and
+  // written through one L2 (a steepest-descent iteration of 24 views of
+  // 512 x 512 0.354 -> 0.331 ms, of 4 views of 1024 x 1024 0.385 -> 0.283)
+  const int nb = gridDim.x, per = nb >> 3;
+  const int b = (nb & 7) == 0 ? (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3)
+                              : (int)blockIdx.x;
+  const int view = b >> (logc - ltc), c0 = (b & (tiles - 1)) << ltc;
+  if (active && !active[view]) return;
   const int col = threadIdx.x & (TC - 1), j = threadIdx.x >> ltc;
   // wave-uniform bases and 32-bit byte offsets (a view is far below 4 GiB)
   float2* vb = data + ((size_t)view << (logr + logc)) + c0;
@@ -382,7 +398,7 @@ struct PrArgs {
   const float2 *y, *D, *v;
   const float* lam;
   float2 *w, *om, *g, *b1, *b2;
-  const int* active;
+  const int* active;  // views to run
   double* scal;  // per view: num, den, alpha, upd
   float nu;
   long long npix, nall;
@@ -516,18 +532,6 @@ __global__ __launch_bounds__(kThreads) void k_pr_update(PrArgs P, double* __rest
   }
 }
 
-// upd = 100 sum|alpha g| / sum|w_new| per view from the partials.
-__global__ void k_pr_update_fin(PrArgs P, const double* __restrict__ part, int n_views) {
-  const int view = blockIdx.x * blockDim.x + threadIdx.x;
-  if (view >= n_views || !P.active[view]) return;
-  double up = 0.0, val = 0.0;
-  for (int b = 0; b < kPrParts; ++b) {
-    up += part[2 * ((size_t)view * kPrParts + b)];
-    val += part[2 * ((size_t)view * kPrParts + b) + 1];
-  }
-  P.scal[4 * view + 3] = 100.0 * up / val;
-}
-
 // Omega = y conj(h) / (|h|^2 + eps), normalised (compute_phase_projection,
 // :10-33); h = H D w in b1.
 __global__ void k_pr_omega(PrArgs P) {
@@ -556,13 +560,182 @@ __global__ __launch_bounds__(kThreads) void k_pr_cost(PrArgs P, double* __restri
   if (threadIdx.x == 0) out[view] = c1 / 2 + (double)P.nu * c2 / 2;
 }
 
-// Stopping test of XT_CmplxProjEst.c:165-169 after iteration j.
-__global__ void k_pr_stop(int n_views, const double* __restrict__ scal, int* __restrict__ active,
-                          int* __restrict__ iters, double thresh, int j) {
-  const int v = blockIdx.x * blockDim.x + threadIdx.x;
-  if (v >= n_views || !active[v]) return;
-  iters[v] = j + 1;
-  if (scal[4 * v + 3] < thresh && j > 1) active[v] = 0;
+// ------------------------------------- steepest descent in fused row passes
+// A transform is a row pass, a column pass and a row pass, and between two
+// transforms there is only elementwise work, so the row passes on both sides
+// of it are one kernel: inverse row FFT, the elementwise step on the values in
+// registers, forward row FFT.  Two of the six transforms of an iteration fall
+// away: H^H is linear, so the gradient's two Hermitian terms are one transform
+// of their difference, and H D w of the phase projection is that of the next
+// iteration's gradient.  Per pixel and iteration 240 bytes move instead of
+// 568: HBM-bound, 24 views of 512 x 512 0.87 -> 0.35 ms per iteration (4.3
+// TB/s over all its passes).
+enum RowStep {
+  kRowsStart,     // D w -> forward
+  kRowsRes,       // inverse = h; conj(Omega) Lambda (Omega h - y) -> forward
+  kRowsGrad,      // inverse = q; g = q conj(D) + nu (w - v), sum 1 |g|^2; D g -> forward
+  kRowsMid,       // inverse = h; conj(Omega) Lambda Omega h -> forward
+  kRowsDen,       // inverse = q; sum 2 Re <g, q conj(D)>
+  kRowsUpd,       // w -= alpha g, sums |alpha g| and |w|; D w -> forward
+  kRowsOmega,     // inverse = h; Omega from h
+  kRowsOmegaRes,  // both kRowsOmega and (with the new Omega) kRowsRes
+};
+
+// Rows of 2^logn >= 8 values, 256 threads on 2048 / 2^logn rows, a row's
+// values in 2^logn / 8 threads' registers.  Rows of views whose active flag is
+// not set are left alone.  part: two FP64 sums per row and wavefront of a row
+// ([row][1 or 2][2]).
+template <int kStep>
+__global__ __launch_bounds__(256) void k_pr_rows(PrArgs P, int logn, int logr, long long nrows,
+                                                 const float2* __restrict__ twg,
+                                                 float2* __restrict__ buf,
+                                                 double* __restrict__ part) {
+  __shared__ float2 s_ex[2048];
+  __shared__ float2 s_tw[kFftMax / 2];
+  constexpr bool kIn = kStep != kRowsStart && kStep != kRowsUpd;
+  constexpr bool kOut = kStep != kRowsDen && kStep != kRowsOmega;
+  constexpr bool kOm = kStep == kRowsOmega || kStep == kRowsOmegaRes;
+  const int n8 = 1 << (logn - 3), S = 256 >> (logn - 3);
+  const int seq = threadIdx.x >> (logn - 3), j = threadIdx.x & (n8 - 1);
+  const long long row = (long long)blockIdx.x * S + seq;
+  const int view = (int)(row >> logr);
+  const bool act = row < nrows && P.active[view] != 0;
+  if (!__syncthreads_or(act)) return;
+  const long long o = act ? (row << logn) + j : j;  // rows left alone read row 0
+  for (int i = threadIdx.x; i < (1 << (logn - 1)); i += 256) s_tw[i] = twg[i];
+  float2 v[8], a[8], b[8], c[8];
+  float l[8];
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const long long q = o + n8 * s;
+    if (kIn) v[s] = buf[q];
+    if (kStep == kRowsStart) v[s] = cmul(P.D[q], P.w[q]);
+    if (kStep == kRowsGrad) {
+      a[s] = P.D[q];
+      b[s] = P.w[q];
+      c[s] = P.v[q];
+    }
+    if (kStep == kRowsDen) {
+      a[s] = P.D[q];
+      b[s] = P.g[q];
+    }
+    if (kStep == kRowsUpd) {
+      a[s] = P.D[q];
+      b[s] = P.w[q];
+      c[s] = P.g[q];
+    }
+    if (kStep == kRowsRes || kStep == kRowsMid) a[s] = P.om[q];
+    if (kStep == kRowsRes || kOm) b[s] = P.y[q];
+    if (kStep == kRowsRes || kStep == kRowsMid || kStep == kRowsOmegaRes) l[s] = P.lam[q];
+  }
+  __syncthreads();
+  if (kIn) fft_reg<true>(v, j, logn, s_tw, s_ex, 1, seq << logn);
+  double s1 = 0.0, s2 = 0.0;
+  const float alpha = kStep == kRowsUpd && act ? (float)P.scal[4 * view + 2] : 0.f;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    const long long q = o + n8 * s;
+    if (kStep == kRowsGrad) {
+      const float2 g = cadd(cmulc(v[s], a[s]), cscale(csub(b[s], c[s]), P.nu));
+      if (act) P.g[q] = g;
+      s1 += (double)g.x * g.x + (double)g.y * g.y;
+      v[s] = cmul(a[s], g);
+    }
+    if (kStep == kRowsDen) {
+      const float2 r = cmulc(v[s], a[s]);
+      s2 += (double)b[s].x * r.x + (double)b[s].y * r.y;
+    }
+    if (kStep == kRowsUpd) {
+      const float2 g = c[s], w = csub(b[s], cscale(g, alpha));
+      if (act) P.w[q] = w;
+      s1 += fabs((double)alpha) * sqrt((double)g.x * g.x + (double)g.y * g.y);
+      s2 += sqrt((double)w.x * w.x + (double)w.y * w.y);
+      v[s] = cmul(a[s], w);
+    }
+    if (kOm) {
+      // Omega = y conj(h) / (|h|^2 + eps), normalised
+      // (compute_phase_projection, XT_PhaseRet.c:10-33)
+      const float2 h = v[s];
+      const float2 t = cscale(cmulc(b[s], h), 1.f / (h.x * h.x + h.y * h.y + FLT_MIN));
+      a[s] = cscale(t, 1.f / (sqrtf(t.x * t.x + t.y * t.y) + FLT_MIN));
+      if (act) P.om[q] = a[s];
+    }
+    if (kStep == kRowsRes || kStep == kRowsOmegaRes || kStep == kRowsMid) {
+      float2 t = cscale(cmul(v[s], a[s]), l[s]);
+      if (kStep != kRowsMid) t = csub(t, cscale(b[s], l[s]));
+      v[s] = cmulc(t, a[s]);
+    }
+  }
+  if (kOut) {
+    fft_reg<false>(v, j, logn, s_tw, s_ex, 1, seq << logn);
+    if (act) {
+#pragma unroll
+      for (int s = 0; s < 8; ++s) buf[o + n8 * s] = v[s];
+    }
+  }
+  if (kStep == kRowsGrad || kStep == kRowsDen || kStep == kRowsUpd) {
+    const int span = n8 < 64 ? n8 : 64;  // a row's lanes within a wavefront
+    for (int d = span / 2; d > 0; d >>= 1) {
+      s1 += __shfl_xor(s1, d);
+      s2 += __shfl_xor(s2, d);
+    }
+    if (act && (j & (span - 1)) == 0) {
+      const size_t k = (size_t)row * (n8 / span) + j / span;
+      if (kStep != kRowsDen) part[2 * k] = s1;
+      if (kStep != kRowsGrad) part[2 * k + 1] = s2;
+    }
+  }
+}
+
+// One block per view: the sum of its k = rows x (1 or 2) row sums, by thread
+// in row order and then by halves (the same order on every call).
+__device__ void view_sum2(const double* __restrict__ part, int view, int k, double& a, double& b) {
+  a = 0.0;
+  b = 0.0;
+  const double* p = part + 2 * (size_t)view * k;
+  for (int i = threadIdx.x; i < k; i += kThreads) {
+    a += p[2 * i];
+    b += p[2 * i + 1];
+  }
+  block_sum2(a, b);
+}
+
+// alpha = num / (den + nu num) (compute_stepsize, XT_PhaseRet.c:133-170),
+// num = |g|^2 and den the sums of kRowsGrad and kRowsDen
+__global__ __launch_bounds__(kThreads) void k_pr_alpha(PrArgs P, const double* __restrict__ part,
+                                                       int k) {
+  const int view = blockIdx.x;
+  if (!P.active[view]) return;
+  double num, den;
+  view_sum2(part, view, k, num, den);
+  if (threadIdx.x == 0) {
+    den += (double)P.nu * num;
+    P.scal[4 * view + 0] = num;
+    P.scal[4 * view + 1] = den;
+    P.scal[4 * view + 2] = num / (den + DBL_MIN);
+  }
+}
+
+// upd = 100 sum|alpha g| / sum|w_new|, the iteration count, and in next the
+// flags of the following iteration (the stopping test of
+// XT_CmplxProjEst.c:165-169 after iteration j)
+__global__ __launch_bounds__(kThreads) void k_pr_upd(PrArgs P, const double* __restrict__ part,
+                                                     int k, double thresh, int j,
+                                                     int* __restrict__ iters,
+                                                     int* __restrict__ next) {
+  const int view = blockIdx.x;
+  if (!P.active[view]) {
+    if (threadIdx.x == 0) next[view] = 0;
+    return;
+  }
+  double up, val;
+  view_sum2(part, view, k, up, val);
+  if (threadIdx.x == 0) {
+    const double upd = 100.0 * up / val;
+    P.scal[4 * view + 3] = upd;
+    iters[view] = j + 1;
+    next[view] = upd < thresh && j > 1 ? 0 : 1;
+  }
 }
 
 // ---------------------------------------------------------------- NMS
@@ -932,8 +1105,11 @@ struct pcmbir_hip_ctx {
   float2* b = nullptr;  // b1 | b2, contiguous: one batched transform of 2 n_views
   float* lam = nullptr;
   int *active = nullptr, *iters = nullptr;
+  int* active2 = nullptr;   // the flags of the following iteration, [n_views]
+  int* h_active = nullptr;  // pinned, [2][n_views]: flags on their way to the host
+  hipEvent_t act_ev[2] = {nullptr, nullptr};
   double *scal = nullptr, *cost = nullptr;
-  double* part = nullptr;  // [n_views][kPrParts][2] partial sums of the step's reductions
+  double* part = nullptr;  // partial sums of the step's reductions
   float nu = 0.f;
   bool problem = false;
   // NMS / ADMM state (estimate_complex_projection)
@@ -965,9 +1141,8 @@ std::vector<float2> twiddles(int n) {
   return t;
 }
 
-// FFT, multiplication by the spectral factor fac [rows][cols], inverse FFT
-// (unnormalised; fac carries 1/N) of nbatch views stored at buf.
-int filter_dev(pcmbir_hip_ctx* c, float2* buf, int nbatch, const float2* fac) {
+// An event pair of the transforms' timing; collect_events sums them.
+int fft_begin(pcmbir_hip_ctx* c) {
   if (c->ev_used == c->ev.size()) {
     hipEvent_t a, b;
     HIP_OK(hipEventCreate(&a));
@@ -975,38 +1150,55 @@ int filter_dev(pcmbir_hip_ctx* c, float2* buf, int nbatch, const float2* fac) {
     c->ev.push_back({a, b});
   }
   HIP_OK(hipEventRecord(c->ev[c->ev_used].first, c->stream));
+  return 0;
+}
+int fft_end(pcmbir_hip_ctx* c, int launches) {
+  HIP_OK(hipGetLastError());
+  HIP_OK(hipEventRecord(c->ev[c->ev_used].second, c->stream));
+  c->ev_used++;
+  c->fft_launches += launches;
+  return 0;
+}
+
+// The column pass of a transform: FFT along rows, times fac, inverse FFT, of
+// the views whose active flag is set (NULL: all).
+void cols_dev(pcmbir_hip_ctx* c, float2* buf, int nbatch, const float2* fac, const int* active) {
+  const bool cols_reg = c->fft_reg && c->logr >= 3;
+  if (cols_reg) {
+    const int ltc = col_tile_reg(c->logr, c->logc, c->col_threads);
+    const unsigned threads = 1u << (ltc + c->logr - 3);
+    const size_t lds = (sizeof(float2) << (ltc + c->logr)) + (sizeof(float2) << (c->logr - 1));
+    hipLaunchKernelGGL(k_fresnel_cols_reg, dim3((unsigned)nbatch << (c->logc - ltc)),
+                       dim3(threads), lds, c->stream, buf, c->logr, c->logc, ltc, c->tw_r, fac, active);
+  } else {
+    const int tiles = c->cols / col_tile(c->logr, c->logc);
+    hipLaunchKernelGGL(k_fresnel_cols, dim3((unsigned)(nbatch * tiles)), dim3(kThreads), 0,
+                       c->stream, buf, c->logr, c->logc, c->tw_r, fac, active);
+  }
+}
+
+// FFT, multiplication by the spectral factor fac [rows][cols], inverse FFT
+// (unnormalised; fac carries 1/N) of nbatch views stored at buf.
+int filter_dev(pcmbir_hip_ctx* c, float2* buf, int nbatch, const float2* fac) {
+  if (fft_begin(c)) return -1;
   const long long nrows = (long long)nbatch * c->rows;
   const unsigned rb = (unsigned)((nrows + (kRowElems >> c->logc) - 1) / (kRowElems >> c->logc));
   // register-resident passes where a sequence holds at least 8 values
-  const bool rows_reg = c->fft_reg && c->logc >= 3, cols_reg = c->fft_reg && c->logr >= 3;
+  const bool rows_reg = c->fft_reg && c->logc >= 3;
   if (rows_reg)
     hipLaunchKernelGGL(k_fft_rows_reg<false>, dim3(rb), dim3(256), 0, c->stream, buf, nrows,
                        c->logc, c->tw_c);
   else
     hipLaunchKernelGGL(k_fft_rows, dim3(rb), dim3(kThreads), 0, c->stream, buf, nrows, c->logc,
                        c->tw_c, 0);
-  if (cols_reg) {
-    const int ltc = col_tile_reg(c->logr, c->logc, c->col_threads);
-    const unsigned threads = 1u << (ltc + c->logr - 3);
-    const size_t lds = (sizeof(float2) << (ltc + c->logr)) + (sizeof(float2) << (c->logr - 1));
-    hipLaunchKernelGGL(k_fresnel_cols_reg, dim3((unsigned)nbatch << (c->logc - ltc)),
-                       dim3(threads), lds, c->stream, buf, c->logr, c->logc, ltc, c->tw_r, fac);
-  } else {
-    const int tiles = c->cols / col_tile(c->logr, c->logc);
-    hipLaunchKernelGGL(k_fresnel_cols, dim3((unsigned)(nbatch * tiles)), dim3(kThreads), 0,
-                       c->stream, buf, c->logr, c->logc, c->tw_r, fac);
-  }
+  cols_dev(c, buf, nbatch, fac, nullptr);
   if (rows_reg)
     hipLaunchKernelGGL(k_fft_rows_reg<true>, dim3(rb), dim3(256), 0, c->stream, buf, nrows,
                        c->logc, c->tw_c);
   else
     hipLaunchKernelGGL(k_fft_rows, dim3(rb), dim3(kThreads), 0, c->stream, buf, nrows, c->logc,
                        c->tw_c, 1);
-  HIP_OK(hipGetLastError());
-  HIP_OK(hipEventRecord(c->ev[c->ev_used].second, c->stream));
-  c->ev_used++;
-  c->fft_launches += 3;
-  return 0;
+  return fft_end(c, 3);
 }
 
 // Fresnel transform (herm = 0: H, 1: H^H) of nbatch views stored at buf.
@@ -1049,12 +1241,56 @@ PrArgs pr_args(pcmbir_hip_ctx* c) {
   return P;
 }
 
+// One fused row pass over every view.
+template <int kStep>
+void rows_dev(pcmbir_hip_ctx* c, const PrArgs& P) {
+  const long long nrows = (long long)c->nv * c->rows;
+  const int S = 256 >> (c->logc - 3);
+  hipLaunchKernelGGL(k_pr_rows<kStep>, dim3((unsigned)((nrows + S - 1) / S)), dim3(256), 0,
+                     c->stream, P, c->logc, c->logr, nrows, c->tw_c, P.b1, c->part);
+}
+
 // Omega = phase projection of the current w (compute_phase_projection,
 // XT_PhaseRet.c:10-33), every view.
 int omega_from_w(pcmbir_hip_ctx* c) {
   const unsigned eb = ew_blocks(c->nall), vb = (unsigned)((c->nv + 255) / 256);
   PrArgs P = pr_args(c);
   hipLaunchKernelGGL(k_fill_int, dim3(vb), dim3(256), 0, c->stream, c->active, c->nv, 1);
+  if (c->fft_reg && c->logc >= 3) {
+    if (fft_begin(c)) return -1;
+    rows_dev<kRowsStart>(c, P);
+    cols_dev(c, P.b1, c->nv, c->fac_h, nullptr);
+    rows_dev<kRowsOmega>(c, P);
+    return fft_end(c, 3);
+  }
+  hipLaunchKernelGGL(k_pr_dmul, dim3(eb), dim3(kThreads), 0, c->stream, P, c->w, P.b1);
+  if (fresnel_dev(c, P.b1, c->nv, 0)) return -1;
+  hipLaunchKernelGGL(k_pr_omega, dim3(eb), dim3(kThreads), 0, c->stream, P);
+  HIP_OK(hipGetLastError());
+  return 0;
+}
+
+// One steepest-descent iteration by separate transforms and elementwise
+// passes: rows shorter than 8 values, or option fft_reg 0.  next: as k_pr_upd.
+int sd_iter_plain(pcmbir_hip_ctx* c, const PrArgs& P) {
+  const unsigned eb = ew_blocks(c->nall), vb = (unsigned)((c->nv + 255) / 256);
+  // gradient (compute_gradient): b1 = H D w, then the two Hermitian passes
+  hipLaunchKernelGGL(k_pr_dmul, dim3(eb), dim3(kThreads), 0, c->stream, P, c->w, P.b1);
+  if (fresnel_dev(c, P.b1, c->nv, 0)) return -1;
+  hipLaunchKernelGGL(k_pr_mid, dim3(eb), dim3(kThreads), 0, c->stream, P, 1);
+  if (fresnel_dev(c, P.b1, 2 * c->nv, 1)) return -1;
+  hipLaunchKernelGGL(k_pr_grad, dim3(eb), dim3(kThreads), 0, c->stream, P);
+  // step size (compute_stepsize)
+  hipLaunchKernelGGL(k_pr_dmul, dim3(eb), dim3(kThreads), 0, c->stream, P, c->g, P.b1);
+  if (fresnel_dev(c, P.b1, c->nv, 0)) return -1;
+  hipLaunchKernelGGL(k_pr_mid, dim3(eb), dim3(kThreads), 0, c->stream, P, 0);
+  if (fresnel_dev(c, P.b1, c->nv, 1)) return -1;
+  hipLaunchKernelGGL(k_pr_step, dim3(c->nv * kPrParts), dim3(kThreads), 0, c->stream, P,
+                     c->part);
+  hipLaunchKernelGGL(k_pr_step_fin, dim3(vb), dim3(256), 0, c->stream, P, c->part, c->nv);
+  hipLaunchKernelGGL(k_pr_update, dim3(c->nv * kPrParts), dim3(kThreads), 0, c->stream, P,
+                     c->part);
+  // phase projection
   hipLaunchKernelGGL(k_pr_dmul, dim3(eb), dim3(kThreads), 0, c->stream, P, c->w, P.b1);
   if (fresnel_dev(c, P.b1, c->nv, 0)) return -1;
   hipLaunchKernelGGL(k_pr_omega, dim3(eb), dim3(kThreads), 0, c->stream, P);
@@ -1064,10 +1300,12 @@ int omega_from_w(pcmbir_hip_ctx* c) {
 
 // The steepest-descent loop over every view whose init_active flag is set
 // (all views when init_active is NULL); per-view stopping as
-// XT_CmplxProjEst.c:165-169.
+// XT_CmplxProjEst.c:165-169.  The host looks at an iteration's flags when the
+// next one has been launched, so that the GPU never waits for it (views that
+// have stopped cost one masked iteration), and not at all where no view can
+// stop (thresh <= 0).
 int sd_loop(pcmbir_hip_ctx* c, int max_iters, double thresh, const int* init_active) {
-  const PrArgs P = pr_args(c);
-  const unsigned eb = ew_blocks(c->nall);
+  PrArgs P = pr_args(c);
   const unsigned vb = (unsigned)((c->nv + 255) / 256);
   if (init_active)
     HIP_OK(hipMemcpyAsync(c->active, init_active, c->nv * sizeof(int), hipMemcpyDeviceToDevice,
@@ -1076,40 +1314,52 @@ int sd_loop(pcmbir_hip_ctx* c, int max_iters, double thresh, const int* init_act
     hipLaunchKernelGGL(k_fill_int, dim3(vb), dim3(256), 0, c->stream, c->active, c->nv, 1);
   hipLaunchKernelGGL(k_fill_int, dim3(vb), dim3(256), 0, c->stream, c->iters, c->nv, 0);
   HIP_OK(hipGetLastError());
-  std::vector<int> act(c->nv);
+  const bool fused = c->fft_reg && c->logc >= 3;
+  const int k = c->rows * (c->logc == 10 ? 2 : 1);  // row sums of a view (k_pr_rows)
+  int *cur = c->active, *next = c->active2;
   for (int j = 0; j < max_iters; ++j) {
-    // gradient (compute_gradient): b1 = H D w, then the two Hermitian passes
-    hipLaunchKernelGGL(k_pr_dmul, dim3(eb), dim3(kThreads), 0, c->stream, P, c->w, P.b1);
-    if (fresnel_dev(c, P.b1, c->nv, 0)) return -1;
-    hipLaunchKernelGGL(k_pr_mid, dim3(eb), dim3(kThreads), 0, c->stream, P, 1);
-    if (fresnel_dev(c, P.b1, 2 * c->nv, 1)) return -1;
-    hipLaunchKernelGGL(k_pr_grad, dim3(eb), dim3(kThreads), 0, c->stream, P);
-    // step size (compute_stepsize)
-    hipLaunchKernelGGL(k_pr_dmul, dim3(eb), dim3(kThreads), 0, c->stream, P, c->g, P.b1);
-    if (fresnel_dev(c, P.b1, c->nv, 0)) return -1;
-    hipLaunchKernelGGL(k_pr_mid, dim3(eb), dim3(kThreads), 0, c->stream, P, 0);
-    if (fresnel_dev(c, P.b1, c->nv, 1)) return -1;
-    hipLaunchKernelGGL(k_pr_step, dim3(c->nv * kPrParts), dim3(kThreads), 0, c->stream, P,
-                       c->part);
-    hipLaunchKernelGGL(k_pr_step_fin, dim3(vb), dim3(256), 0, c->stream, P, c->part, c->nv);
-    hipLaunchKernelGGL(k_pr_update, dim3(c->nv * kPrParts), dim3(kThreads), 0, c->stream, P,
-                       c->part);
-    hipLaunchKernelGGL(k_pr_update_fin, dim3(vb), dim3(256), 0, c->stream, P, c->part, c->nv);
-    // phase projection
-    hipLaunchKernelGGL(k_pr_dmul, dim3(eb), dim3(kThreads), 0, c->stream, P, c->w, P.b1);
-    if (fresnel_dev(c, P.b1, c->nv, 0)) return -1;
-    hipLaunchKernelGGL(k_pr_omega, dim3(eb), dim3(kThreads), 0, c->stream, P);
-    hipLaunchKernelGGL(k_pr_stop, dim3(vb), dim3(256), 0, c->stream, c->nv, c->scal, c->active,
-                       c->iters, thresh, j);
-    HIP_OK(hipGetLastError());
-    HIP_OK(hipMemcpyAsync(act.data(), c->active, c->nv * sizeof(int), hipMemcpyDeviceToHost,
-                          c->stream));
-    if (collect_events(c)) return -1;
-    bool any = false;
-    for (int a : act) any = any || a;
-    if (!any) break;
+    P.active = cur;
+    if (fused) {
+      if (fft_begin(c)) return -1;
+      if (j == 0) {
+        rows_dev<kRowsStart>(c, P);
+        cols_dev(c, P.b1, c->nv, c->fac_h, cur);
+        rows_dev<kRowsRes>(c, P);
+      }
+      // gradient, then the step size, the update and the phase projection
+      cols_dev(c, P.b1, c->nv, c->fac_hh, cur);
+      rows_dev<kRowsGrad>(c, P);
+      cols_dev(c, P.b1, c->nv, c->fac_h, cur);
+      rows_dev<kRowsMid>(c, P);
+      cols_dev(c, P.b1, c->nv, c->fac_hh, cur);
+      rows_dev<kRowsDen>(c, P);
+      hipLaunchKernelGGL(k_pr_alpha, dim3(c->nv), dim3(kThreads), 0, c->stream, P, c->part, k);
+      rows_dev<kRowsUpd>(c, P);
+      hipLaunchKernelGGL(k_pr_upd, dim3(c->nv), dim3(kThreads), 0, c->stream, P, c->part, k,
+                         thresh, j, c->iters, next);
+      cols_dev(c, P.b1, c->nv, c->fac_h, cur);
+      if (j + 1 < max_iters)
+        rows_dev<kRowsOmegaRes>(c, P);
+      else
+        rows_dev<kRowsOmega>(c, P);
+      if (fft_end(c, j == 0 ? 12 : 9)) return -1;
+    } else {
+      if (sd_iter_plain(c, P)) return -1;
+      hipLaunchKernelGGL(k_pr_upd, dim3(c->nv), dim3(kThreads), 0, c->stream, P, c->part,
+                         kPrParts, thresh, j, c->iters, next);
+      HIP_OK(hipGetLastError());
+    }
+    std::swap(cur, next);
+    if (!(thresh > 0)) continue;
+    HIP_OK(hipMemcpyAsync(c->h_active + (j & 1) * c->nv, cur, c->nv * sizeof(int),
+                          hipMemcpyDeviceToHost, c->stream));
+    HIP_OK(hipEventRecord(c->act_ev[j & 1], c->stream));
+    if (j < 3) continue;  // no view stops before iteration 2
+    HIP_OK(hipEventSynchronize(c->act_ev[(j - 1) & 1]));
+    const int* a = c->h_active + ((j - 1) & 1) * c->nv;
+    if (std::all_of(a, a + c->nv, [](int f) { return f == 0; })) break;
   }
-  return 0;
+  return collect_events(c);
 }
 
 int alloc_nms_state(pcmbir_hip_ctx* c) {
@@ -1214,9 +1464,13 @@ void pcmbir_hip_destroy(pcmbir_hip_ctx* c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   void* bufs[] = {c->tw_r, c->tw_c, c->fac_h, c->fac_hh, c->fac_pag, c->y, c->D, c->v, c->w, c->om,
                   c->g, c->b, c->lam, c->active, c->iters, c->scal, c->cost, c->part,
-                  c->zr, c->zi, c->res, c->vd, c->wold, c->pix_iters, c->admm, c->ar, c->ai};
+                  c->zr, c->zi, c->res, c->vd, c->wold, c->pix_iters, c->admm, c->ar, c->ai,
+                  c->active2};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
+  if (c->h_active) (void)hipHostFree(c->h_active);
+  for (auto& e : c->act_ev)
+    if (e) (void)hipEventDestroy(e);
   for (auto& pr : c->ev) {
     (void)hipEventDestroy(pr.first);
     (void)hipEventDestroy(pr.second);
@@ -1243,8 +1497,11 @@ int pcmbir_hip_set_phase_problem(pcmbir_hip_ctx* c, const float* y, const float*
         dev_alloc(&c->w, c->nall) || dev_alloc(&c->om, c->nall) || dev_alloc(&c->g, c->nall) ||
         dev_alloc(&c->lam, c->nall) || dev_alloc(&c->active, c->nv) ||
         dev_alloc(&c->iters, c->nv) || dev_alloc(&c->scal, 4 * (size_t)c->nv) ||
-        dev_alloc(&c->cost, c->nv) || dev_alloc(&c->part, 2 * (size_t)kPrParts * c->nv))
+        dev_alloc(&c->cost, c->nv) || dev_alloc(&c->active2, c->nv) ||
+        dev_alloc(&c->part, (size_t)c->nv * std::max(2 * kPrParts, 4 * c->rows)))
       return -1;
+    HIP_OK(hipHostMalloc((void**)&c->h_active, 2 * (size_t)c->nv * sizeof(int)));
+    for (auto& e : c->act_ev) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   }
   const size_t cb = (size_t)c->nall * sizeof(float2);
   HIP_OK(hipMemcpyAsync(c->y, y, cb, hipMemcpyHostToDevice, c->stream));
