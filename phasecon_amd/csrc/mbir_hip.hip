@@ -34,6 +34,7 @@
 
 #include "mbir_hip.h"
 #include "mbir_engine.h"
+#include "copy_out.h"
 #include "pow64.h"
 
 namespace {
@@ -2622,6 +2623,7 @@ int dev_alloc(T** p, size_t n) {
 }  // namespace
 
 struct mbir_hip_ctx {
+  phasecon::CopyOut copy_out;
   mbir_hip_geom g;
   DevGeom G;
   SwGeom SG;
@@ -3085,8 +3087,7 @@ int mbir_hip_get_object(mbir_hip_ctx* c, float* x) {
   hipLaunchKernelGGL(k_from_colmajor, dim3(blocks), dim3(256), 0, c->stream, c->g.N_time,
                      c->g.N_z, c->ncol, c->d_x, c->d_stage);
   HIP_OK(hipGetLastError());
-  HIP_OK(hipMemcpyAsync(x, c->d_stage, c->nvox * sizeof(float), hipMemcpyDeviceToHost,
-                        c->stream));
+  HIP_OK(c->copy_out(x, c->d_stage, c->nvox * sizeof(float), c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -3148,7 +3149,7 @@ int mbir_hip_init_error(mbir_hip_ctx* c) {
 
 int mbir_hip_get_error(mbir_hip_ctx* c, float* e) {
   if (!c || !e) return fail("null argument");
-  HIP_OK(hipMemcpyAsync(e, c->d_e, c->nsino * sizeof(float), hipMemcpyDeviceToHost, c->stream));
+  HIP_OK(c->copy_out(e, c->d_e, c->nsino * sizeof(float), c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -3169,8 +3170,7 @@ int mbir_hip_forward_project(mbir_hip_ctx* c, const float* x, float* ax) {
                      c->g.N_z, c->ncol, c->d_stage, c->d_stage2);
   HIP_OK(hipGetLastError());
   if (run_fwdproj(c, 2, c->d_stage2, c->d_stage)) return -1;
-  HIP_OK(hipMemcpyAsync(ax, c->d_stage, c->nsino * sizeof(float), hipMemcpyDeviceToHost,
-                        c->stream));
+  HIP_OK(c->copy_out(ax, c->d_stage, c->nsino * sizeof(float), c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -3187,8 +3187,7 @@ int mbir_hip_backproject(mbir_hip_ctx* c, const float* v, float* bt) {
   hipLaunchKernelGGL(k_from_colmajor, dim3(blocks), dim3(256), 0, c->stream, c->g.N_time,
                      c->g.N_z, c->ncol, c->d_stage2, c->d_stage);
   HIP_OK(hipGetLastError());
-  HIP_OK(hipMemcpyAsync(bt, c->d_stage, c->nvox * sizeof(float), hipMemcpyDeviceToHost,
-                        c->stream));
+  HIP_OK(c->copy_out(bt, c->d_stage, c->nvox * sizeof(float), c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -3208,8 +3207,7 @@ int mbir_hip_bp_normalized(mbir_hip_ctx* c, float* out) {
   hipLaunchKernelGGL(k_from_colmajor, dim3(blocks), dim3(256), 0, c->stream, c->g.N_time,
                      c->g.N_z, c->ncol, c->d_stage2, c->d_stage);
   HIP_OK(hipGetLastError());
-  HIP_OK(hipMemcpyAsync(out, c->d_stage, c->nvox * sizeof(float), hipMemcpyDeviceToHost,
-                        c->stream));
+  HIP_OK(c->copy_out(out, c->d_stage, c->nvox * sizeof(float), c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -3244,8 +3242,7 @@ int mbir_hip_fbp(mbir_hip_ctx* c, float* out) {
   hipLaunchKernelGGL(k_from_colmajor, dim3(bo), dim3(256), 0, c->stream, c->g.N_time, c->g.N_z,
                      c->ncol, c->d_stage2, c->d_stage);
   HIP_OK(hipGetLastError());
-  HIP_OK(hipMemcpyAsync(out, c->d_stage, c->nvox * sizeof(float), hipMemcpyDeviceToHost,
-                        c->stream));
+  HIP_OK(c->copy_out(out, c->d_stage, c->nvox * sizeof(float), c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -3954,8 +3951,7 @@ int mbir_hip_pc_get_objects(mbir_hip_ctx* c, float* delta, float* beta) {
   hipLaunchKernelGGL(k_from_colmajor, dim3(blocks), dim3(256), 0, c->stream, c->g.N_time,
                      c->g.N_z, c->ncol, c->d_x2, c->d_stage);
   HIP_OK(hipGetLastError());
-  HIP_OK(hipMemcpyAsync(beta, c->d_stage, c->nvox * sizeof(float), hipMemcpyDeviceToHost,
-                        c->stream));
+  HIP_OK(c->copy_out(beta, c->d_stage, c->nvox * sizeof(float), c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -3980,10 +3976,8 @@ int mbir_hip_pc_init_error(mbir_hip_ctx* c, const float* target_delta, const flo
 int mbir_hip_pc_get_error(mbir_hip_ctx* c, float* e_delta, float* e_beta) {
   if (!c || !e_delta || !e_beta) return fail("null argument");
   if (!c->pc) return fail("tomographic mode not enabled (mbir_hip_pc_enable)");
-  HIP_OK(hipMemcpyAsync(e_delta, c->d_e, c->nsino * sizeof(float), hipMemcpyDeviceToHost,
-                        c->stream));
-  HIP_OK(hipMemcpyAsync(e_beta, c->d_e2, c->nsino * sizeof(float), hipMemcpyDeviceToHost,
-                        c->stream));
+  HIP_OK(c->copy_out(e_delta, c->d_e, c->nsino * sizeof(float), c->stream));
+  HIP_OK(c->copy_out(e_beta, c->d_e2, c->nsino * sizeof(float), c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -4138,8 +4132,8 @@ int mbir_hip_pc_admm_state(mbir_hip_ctx* c, int32_t which, float* delta, float* 
   if (which < 0 || which > 2) return fail("which must be 0 (Z), 1 (V) or 2 (P)");
   const float* src = which == 0 ? c->d_pz : which == 1 ? c->d_pv : c->d_pp;
   const size_t n = c->nsino;
-  HIP_OK(hipMemcpyAsync(delta, src, n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
-  HIP_OK(hipMemcpyAsync(beta, src + n, n * sizeof(float), hipMemcpyDeviceToHost, c->stream));
+  HIP_OK(c->copy_out(delta, src, n * sizeof(float), c->stream));
+  HIP_OK(c->copy_out(beta, src + n, n * sizeof(float), c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }

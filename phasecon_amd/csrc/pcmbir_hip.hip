@@ -31,6 +31,7 @@
 #include <vector>
 
 #include "pcmbir_hip.h"
+#include "copy_out.h"
 #include "pow64.h"
 
 namespace {
@@ -1135,6 +1136,7 @@ int ilog2(int v) {
 }  // namespace
 
 struct pcmbir_hip_ctx {
+  phasecon::CopyOut copy_out;
   int nv = 0, rows = 0, cols = 0, logr = 0, logc = 0;
   long long npix = 0, nall = 0;
   hipStream_t stream = nullptr;
@@ -1533,7 +1535,7 @@ int pcmbir_hip_fresnel(pcmbir_hip_ctx* c, int32_t herm, const float* x, float* y
   const size_t bytes = (size_t)c->nall * sizeof(float2);
   HIP_OK(hipMemcpyAsync(c->b, x, bytes, hipMemcpyHostToDevice, c->stream));
   if (fresnel_dev(c, c->b, c->nv, herm != 0)) return -1;
-  HIP_OK(hipMemcpyAsync(y, c->b, bytes, hipMemcpyDeviceToHost, c->stream));
+  HIP_OK(c->copy_out(y, c->b, bytes, c->stream));
   return collect_events(c);
 }
 
@@ -1591,8 +1593,8 @@ int pcmbir_hip_get_phase_state(pcmbir_hip_ctx* c, float* w, float* omega) {
   if (!c || !w || !omega) return fail("null argument");
   if (!c->problem) return fail("no phase problem set");
   const size_t cb = (size_t)c->nall * sizeof(float2);
-  HIP_OK(hipMemcpyAsync(w, c->w, cb, hipMemcpyDeviceToHost, c->stream));
-  HIP_OK(hipMemcpyAsync(omega, c->om, cb, hipMemcpyDeviceToHost, c->stream));
+  HIP_OK(c->copy_out(w, c->w, cb, c->stream));
+  HIP_OK(c->copy_out(omega, c->om, cb, c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -1691,8 +1693,8 @@ int pcmbir_hip_nms_pass(pcmbir_hip_ctx* c, double* zr, double* zi, const float* 
   const unsigned vb = (unsigned)((c->nv + 255) / 256);
   hipLaunchKernelGGL(k_fill_int, dim3(vb), dim3(256), 0, c->stream, c->admm, c->nv, 1);
   if (nms_pass_dev(c, c->wold, c->vd, c->admm)) return -1;
-  HIP_OK(hipMemcpyAsync(zr, c->zr, db, hipMemcpyDeviceToHost, c->stream));
-  HIP_OK(hipMemcpyAsync(zi, c->zi, db, hipMemcpyDeviceToHost, c->stream));
+  HIP_OK(c->copy_out(zr, c->zr, db, c->stream));
+  HIP_OK(c->copy_out(zi, c->zi, db, c->stream));
   std::vector<int> it(c->nall);
   HIP_OK(hipMemcpyAsync(it.data(), c->pix_iters, c->nall * sizeof(int), hipMemcpyDeviceToHost,
                         c->stream));
@@ -1763,8 +1765,8 @@ int pcmbir_hip_estimate(pcmbir_hip_ctx* c, double* zr, double* zi, int32_t pret_
   }
   if (iters)
     for (int v = 0; v < c->nv; ++v) iters[v] = its[v];
-  HIP_OK(hipMemcpyAsync(zr, c->zr, db, hipMemcpyDeviceToHost, c->stream));
-  HIP_OK(hipMemcpyAsync(zi, c->zi, db, hipMemcpyDeviceToHost, c->stream));
+  HIP_OK(c->copy_out(zr, c->zr, db, c->stream));
+  HIP_OK(c->copy_out(zi, c->zi, db, c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -1776,7 +1778,7 @@ int pcmbir_hip_get_dual(pcmbir_hip_ctx* c, float* v) {
     memset(v, 0, cb);
     return 0;
   }
-  HIP_OK(hipMemcpyAsync(v, c->vd, cb, hipMemcpyDeviceToHost, c->stream));
+  HIP_OK(c->copy_out(v, c->vd, cb, c->stream));
   HIP_OK(hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -1816,8 +1818,8 @@ int pcmbir_hip_paganin(pcmbir_hip_ctx* c, const float* y, const float* D,
   hipLaunchKernelGGL(k_pag_post, dim3(eb), dim3(kThreads), 0, c->stream, c->b, c->nall,
                      delta_over_beta, c->zr, c->zi);
   HIP_OK(hipGetLastError());
-  HIP_OK(hipMemcpyAsync(zr, c->zr, db, hipMemcpyDeviceToHost, c->stream));
-  HIP_OK(hipMemcpyAsync(zi, c->zi, db, hipMemcpyDeviceToHost, c->stream));
+  HIP_OK(c->copy_out(zr, c->zr, db, c->stream));
+  HIP_OK(c->copy_out(zi, c->zi, db, c->stream));
   return collect_events(c);
 }
 

@@ -36,6 +36,7 @@
 #include <string>
 #include <vector>
 
+#include "copy_out.h"
 #include "unet_hip.h"
 
 namespace {
@@ -914,6 +915,7 @@ int launch_dw(hipStream_t s, const Chan& g, const ConvIn& in, float* dw, float* 
 
 // ------------------------------------------------------------------ network
 struct unet_ctx {
+  phasecon::CopyOut copy_out;
   hipStream_t s = nullptr;
   int c = 16, cin = 1;  // base channels, input channels
   Layer L[kLayers];
@@ -1201,7 +1203,7 @@ int unet_forward(unet_ctx* c, int32_t N, int32_t D, int32_t H, int32_t W, const 
                  float* y) {
   if (!c || !x || !y) return fail("null argument");
   if (set_shape(c, N, D, H, W) || upload_pair(c, x, nullptr) || forward(c, true)) return -1;
-  HIP_OK(hipMemcpyAsync(y, c->o32, c->V1 * sizeof(float), hipMemcpyDeviceToHost, c->s));
+  HIP_OK(c->copy_out(y, c->o32, c->V1 * sizeof(float), c->s));
   HIP_OK(hipStreamSynchronize(c->s));
   return 0;
 }
