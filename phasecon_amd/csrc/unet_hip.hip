@@ -946,26 +946,15 @@ namespace {
 
 constexpr int kLossBlocks = 256;
 
-int alloc_act(unet_ctx* c, u16** p, long long n) {
-  if (dalloc(p, (size_t)n)) return -1;
-  c->acts.push_back(*p);
-  return 0;
+template <typename T>
+int alloc_act(unet_ctx* c, T** p, long long n) {
+  const int rc = dalloc(p, (size_t)n);
+  if (*p) c->acts.push_back(*p);
+  return rc;
 }
 
-int set_shape(unet_ctx* c, int N, int D, int H, int W) {
-  if (N == c->N && D == c->D && H == c->H && W == c->W) return 0;
-  if (N < 1 || D < 4 || H < 4 || W < 64 || D % 4 || H % 4 || W % 64)
-    return fail("volume must have D, H divisible by 4 and W divisible by 64");
-  HIP_OK(hipStreamSynchronize(c->s));
-  c->free_acts();
-  c->N = N;
-  c->D = D;
-  c->H = H;
-  c->W = W;
+int alloc_shape(unet_ctx* c, int N, int D, int H, int W) {
   const long long V1 = (long long)N * D * H * W, V2 = V1 / 8, V3 = V1 / 64;
-  c->V1 = V1;
-  c->V2 = V2;
-  c->V3 = V3;
   const int c1 = c->c, c2 = 2 * c->c, c3 = 4 * c->c;
   u16** bufs1[] = {&c->A1, &c->A5, &c->B5, &c->GB5, &c->GA5, &c->GA1};
   for (u16** b : bufs1)
@@ -989,13 +978,33 @@ int set_shape(unet_ctx* c, int N, int D, int H, int W) {
     part = std::max(part, dw_partial(dw_tiles(N, D >> sh, H >> sh, W >> sh), c->L[i].cin,
                                      c->L[i].cout));
   }
-  if (dalloc(&c->dwpart, part)) return -1;
-  c->acts.push_back(c->dwpart);
+  if (alloc_act(c, &c->dwpart, (long long)part)) return -1;
   float** f32s[] = {&c->x32, &c->t32, &c->o32};
-  for (float** b : f32s) {
-    if (dalloc(b, (size_t)V1 * (b == &c->x32 ? c->cin : 1))) return -1;
-    c->acts.push_back(*b);
+  for (float** b : f32s)
+    if (alloc_act(c, b, V1 * (b == &c->x32 ? c->cin : 1))) return -1;
+  return 0;
+}
+
+// The activation buffers of a shape.  The context holds the shape only once
+// all of them are there: a call after a failed one allocates again.
+int set_shape(unet_ctx* c, int N, int D, int H, int W) {
+  if (N == c->N && D == c->D && H == c->H && W == c->W) return 0;
+  if (N < 1 || D < 4 || H < 4 || W < 64 || D % 4 || H % 4 || W % 64)
+    return fail("volume must have D, H divisible by 4 and W divisible by 64");
+  HIP_OK(hipStreamSynchronize(c->s));
+  c->free_acts();
+  c->N = 0;
+  if (alloc_shape(c, N, D, H, W)) {
+    c->free_acts();
+    return -1;
   }
+  c->N = N;
+  c->D = D;
+  c->H = H;
+  c->W = W;
+  c->V1 = (long long)N * D * H * W;
+  c->V2 = c->V1 / 8;
+  c->V3 = c->V1 / 64;
   return 0;
 }
 
