@@ -1127,6 +1127,18 @@ int dev_alloc(T** p, size_t n) {
   return 0;
 }
 
+// All buffers of a group (pointer, count, pointer, count, ...) or none: its
+// first pointer tells whether the group is there.
+inline int dev_alloc_all() { return 0; }
+template <typename T, typename... R>
+int dev_alloc_all(T** p, size_t n, R... rest) {
+  if (dev_alloc(p, n)) return -1;
+  if (dev_alloc_all(rest...) == 0) return 0;
+  (void)hipFree(*p);
+  *p = nullptr;
+  return -1;
+}
+
 int ilog2(int v) {
   int l = 0;
   while ((1 << l) < v) ++l;
@@ -1412,11 +1424,9 @@ int sd_loop(pcmbir_hip_ctx* c, int max_iters, double thresh, const int* init_act
 
 int alloc_nms_state(pcmbir_hip_ctx* c) {
   if (c->zr) return 0;
-  if (dev_alloc(&c->zr, c->nall) || dev_alloc(&c->zi, c->nall) || dev_alloc(&c->res, 3 * (size_t)c->nv) ||
-      dev_alloc(&c->vd, c->nall) || dev_alloc(&c->wold, c->nall) ||
-      dev_alloc(&c->pix_iters, c->nall) || dev_alloc(&c->admm, c->nv))
-    return -1;
-  return 0;
+  const size_t n = c->nall, nv = c->nv;
+  return dev_alloc_all(&c->zr, n, &c->zi, n, &c->res, 3 * nv, &c->vd, n, &c->wold, n,
+                       &c->pix_iters, n, &c->admm, nv);
 }
 
 // The four colours of an NMS pass over the active views (admm mask).
@@ -1543,16 +1553,12 @@ int pcmbir_hip_set_phase_problem(pcmbir_hip_ctx* c, const float* y, const float*
                                  const float* lambda, const float* v, const float* w,
                                  const float* omega, double nu) {
   if (!c || !y || !D || !lambda || !v || !w) return fail("null argument");
-  if (!c->y) {
-    if (dev_alloc(&c->y, c->nall) || dev_alloc(&c->D, c->nall) || dev_alloc(&c->v, c->nall) ||
-        dev_alloc(&c->w, c->nall) || dev_alloc(&c->om, c->nall) || dev_alloc(&c->g, c->nall) ||
-        dev_alloc(&c->lam, c->nall) || dev_alloc(&c->active, c->nv) ||
-        dev_alloc(&c->iters, c->nv) || dev_alloc(&c->scal, 4 * (size_t)c->nv) ||
-        dev_alloc(&c->cost, c->nv) || dev_alloc(&c->active2, c->nv) ||
-        dev_alloc(&c->part, (size_t)c->nv * std::max(3 * kPrParts, 4 * c->rows)))
-      return -1;
-
-  }
+  const size_t n = c->nall, nv = c->nv;
+  if (!c->y && dev_alloc_all(&c->y, n, &c->D, n, &c->v, n, &c->w, n, &c->om, n, &c->g, n, &c->lam,
+                             n, &c->active, nv, &c->active2, nv, &c->iters, nv, &c->scal, 4 * nv,
+                             &c->cost, nv, &c->part,
+                             nv * std::max(3 * kPrParts, 4 * c->rows)))
+    return -1;
   const size_t cb = (size_t)c->nall * sizeof(float2);
   HIP_OK(hipMemcpyAsync(c->y, y, cb, hipMemcpyHostToDevice, c->stream));
   HIP_OK(hipMemcpyAsync(c->D, D, cb, hipMemcpyHostToDevice, c->stream));
@@ -1668,7 +1674,7 @@ int pcmbir_hip_set_tomo_target(pcmbir_hip_ctx* c, double mu, const double* a_mag
     return 0;
   }
   if (!(mu > 0)) return fail("mu must be positive");
-  if (!c->ar && (dev_alloc(&c->ar, c->nall) || dev_alloc(&c->ai, c->nall))) return -1;
+  if (!c->ar && dev_alloc_all(&c->ar, (size_t)c->nall, &c->ai, (size_t)c->nall)) return -1;
   const size_t db = (size_t)c->nall * sizeof(double);
   HIP_OK(hipMemcpyAsync(c->ar, a_mag, db, hipMemcpyHostToDevice, c->stream));
   HIP_OK(hipMemcpyAsync(c->ai, a_phase, db, hipMemcpyHostToDevice, c->stream));

@@ -143,6 +143,22 @@ hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t*, const void*) {
   return hipErrorInvalidValue;  // plain host memory
 }
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) {
+  *v = 160 * 1024;  // the only one asked for: LDS per workgroup
+  return hipSuccess;
+}
+hipError_t hipGetSymbolAddress(void** p, const void* s) {
+  *p = const_cast<void*>(s);
+  return hipSuccess;
+}
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipErrorNotSupported; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t*) { return hipErrorNotSupported; }
+hipError_t hipGraphInstantiate(hipGraphExec_t*, hipGraph_t, hipGraphNode_t*, char*, size_t) {
+  return hipErrorNotSupported;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipErrorNotSupported; }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
 
 // ------------------------------------------------------------ compiler's side
 void** __hipRegisterFatBinary(const void*) {
