@@ -2635,6 +2635,18 @@ int dev_alloc(T** p, size_t n) {
   return 0;
 }
 
+// All buffers of a group (pointer, count, pointer, count, ...) or none: its
+// first pointer tells whether the group is there.
+inline int dev_alloc_all() { return 0; }
+template <typename T, typename... R>
+int dev_alloc_all(T** p, size_t n, R... rest) {
+  if (dev_alloc(p, n)) return -1;
+  if (dev_alloc_all(rest...) == 0) return 0;
+  (void)hipFree(*p);
+  *p = nullptr;
+  return -1;
+}
+
 }  // namespace
 
 struct mbir_hip_ctx {
@@ -2745,6 +2757,7 @@ int ev_collect(mbir_hip_ctx* c) {
 
 int ensure_partial(mbir_hip_ctx* c, size_t n) {
   if (n <= c->partial_cap) return 0;
+  c->partial_cap = 0;
   if (c->d_partial) HIP_OK(hipFree(c->d_partial));
   if (dev_alloc(&c->d_partial, n)) return -1;
   c->partial_cap = n;
@@ -2772,11 +2785,13 @@ int build_tiles(mbir_hip_ctx* c) {
     launch.insert(launch.end(), order[k].begin(), order[k].end());
   }
   c->launch_off[4] = (int)launch.size();
-  if (c->d_tile_ptr) HIP_OK(hipFree(c->d_tile_ptr));
-  if (c->d_tile_cols) HIP_OK(hipFree(c->d_tile_cols));
-  if (c->d_launch_tiles) HIP_OK(hipFree(c->d_launch_tiles));
-  if (dev_alloc(&c->d_tile_ptr, ptr.size()) || dev_alloc(&c->d_tile_cols, cols.size()) ||
-      dev_alloc(&c->d_launch_tiles, launch.size()))
+  c->tiles_for = -1;
+  for (int** p : {&c->d_tile_ptr, &c->d_tile_cols, &c->d_launch_tiles}) {
+    if (*p) HIP_OK(hipFree(*p));
+    *p = nullptr;
+  }
+  if (dev_alloc_all(&c->d_tile_ptr, ptr.size(), &c->d_tile_cols, cols.size(), &c->d_launch_tiles,
+                    launch.size()))
     return -1;
   HIP_OK(hipMemcpy(c->d_tile_ptr, ptr.data(), ptr.size() * sizeof(int), hipMemcpyHostToDevice));
   if (!cols.empty())
@@ -3037,7 +3052,7 @@ int mbir_hip_set_option(mbir_hip_ctx* c, const char* key, double value) {
     if (value != 0 && value != 1) return fail("nhicd must be 0 or 1");
     if (value == 1 && !c->d_mag) {
       const size_t nm = (size_t)c->ncol * c->g.N_time;
-      if (dev_alloc(&c->d_mag, nm) || dev_alloc(&c->d_vsc, nm)) return -1;
+      if (dev_alloc_all(&c->d_mag, nm, &c->d_vsc, nm)) return -1;
       HIP_OK(hipMemset(c->d_mag, 0, nm * sizeof(float)));
     }
     c->nh = value == 1;
@@ -3126,9 +3141,7 @@ int mbir_hip_object_snapshot(mbir_hip_ctx* c, int32_t restore) {
 int mbir_hip_build_amatrix(mbir_hip_ctx* c) {
   if (!c) return fail("null context");
   const size_t n = (size_t)c->ncol * c->nslots;
-  if (!c->d_afirst) {
-    if (dev_alloc(&c->d_afirst, n) || dev_alloc(&c->d_aval, n * c->G.W)) return -1;
-  }
+  if (!c->d_afirst && dev_alloc_all(&c->d_afirst, n, &c->d_aval, n * c->G.W)) return -1;
   if (n == 0) return 0;
   if (ev_begin(c, MBIR_K_AMATRIX)) return -1;
   hipLaunchKernelGGL(k_amatrix, dim3((unsigned)((n + 255) / 256)), dim3(256),
@@ -3136,7 +3149,7 @@ int mbir_hip_build_amatrix(mbir_hip_ctx* c) {
                      c->d_sin, c->d_frame_views, c->d_afirst, c->d_aval);
   if (c->afp16) {
     if (!c->d_aval16 &&
-        (dev_alloc(&c->d_aval16, n * c->G.W) || dev_alloc(&c->d_ascale, (size_t)c->ncol)))
+        dev_alloc_all(&c->d_aval16, n * c->G.W, &c->d_ascale, (size_t)c->ncol))
       return -1;
     hipLaunchKernelGGL(k_aquant, dim3((unsigned)((c->ncol + 3) / 4)), dim3(256), 0, c->stream,
                        c->ncol, c->nslots * c->G.W, c->d_aval, c->d_aval16, c->d_ascale);
@@ -3913,7 +3926,7 @@ int mbir_hip_pc_enable(mbir_hip_ctx* c, const mbir_hip_pc_prior* pr) {
   if (pr->q != 2.0) return fail("q must be 2 (the qGGMRF of the tomographic kernels)");
   if (pr->mu <= 0 || pr->wavenumber <= 0) return fail("mu and the wavenumber must be positive");
   if (c->g.N_z > kNZPc) return fail("the tomographic sweep takes at most 256 voxels per column");
-  if (!c->d_x2 && (dev_alloc(&c->d_x2, c->nvox) || dev_alloc(&c->d_e2, c->nsino))) return -1;
+  if (!c->d_x2 && dev_alloc_all(&c->d_x2, c->nvox, &c->d_e2, c->nsino)) return -1;
   HIP_OK(hipMemset(c->d_x2, 0, c->nvox * sizeof(float)));
   HIP_OK(hipMemset(c->d_e2, 0, c->nsino * sizeof(float)));
   PcTab& P = c->ptab;
@@ -4061,9 +4074,8 @@ int mbir_hip_pc_admm_init(mbir_hip_ctx* c, const double* z_delta, const double* 
   if (!c->pc) return fail("tomographic mode not enabled (mbir_hip_pc_enable)");
   if (!c->a_built) return fail("A not built");
   const size_t n = c->nsino;
-  if (!c->d_pz && (dev_alloc(&c->d_pz, 2 * n) || dev_alloc(&c->d_pv, 2 * n) ||
-                   dev_alloc(&c->d_pp, 2 * n) || dev_alloc(&c->d_pk, n) ||
-                   dev_alloc(&c->d_pdbl, n)))
+  if (!c->d_pz && dev_alloc_all(&c->d_pz, 2 * n, &c->d_pv, 2 * n, &c->d_pp, 2 * n, &c->d_pk, n,
+                                &c->d_pdbl, n))
     return -1;
   const double k = (double)c->ptab.kw;
   const double* zs[2] = {z_delta, z_beta};

@@ -1,0 +1,111 @@
+"""The MBIR library's host side against a stand-in for the HIP runtime
+(hip_stub.py): what a failed allocation leaves behind."""
+import os
+
+import numpy as np
+import pytest
+
+import hip_stub
+
+pytestmark = pytest.mark.skipif(not os.path.exists(hip_stub.HIPCC), reason="no hipcc")
+
+
+@pytest.fixture
+def L(monkeypatch):
+    return hip_stub.use(monkeypatch)
+
+
+def _scan():
+    from phasecon_amd.synth import geometry_scan
+    return geometry_scan(4, 16, 6)
+
+
+def _stage(**kw):
+    from phasecon_amd.mbir import Stage
+    return Stage(_scan(), **kw)
+
+
+def _built():
+    st = _stage()
+    st.build_amatrix()
+    return st
+
+
+def _half():
+    st = _built()
+    st.option("afp16", 1)
+    return st
+
+
+def _swept():
+    st = _built()
+    st.icd(1, 1)
+    st.option("tile", 4)
+    return st
+
+
+def _tomo():
+    from phasecon_amd.mbir import TomoStage, tomo_prior
+    p = tomo_prior((2e-7, 1e-3, 0.01, 0.01), (2e-10, 1e-3, 0.01, 0.01), 1, 6.0, 1.0,
+                   delta_over_beta=50.0, mu=0.5, alpha=1.5)
+    st = TomoStage(_scan(), p)
+    z = np.zeros(st.shape_e, np.float32)
+    st.init_errors(z, z)
+    return st
+
+
+def _admm(st):
+    z = np.zeros(st.shape_e)
+    st.admm_init(z, z)
+
+
+# every call that allocates a group of buffers: the context it is made on, how
+# many there are, and a kernel that reads them
+@pytest.mark.parametrize("make,call,n,kernel", [
+    (_stage, lambda st: st.build_amatrix(), 2, "k_amatrix"),
+    (_half, lambda st: st.build_amatrix(), 2, "k_aquant"),
+    (_built, lambda st: st.option("nhicd", 1), 2, "k_vsc"),
+    (_built, lambda st: st.icd(1, 1), 3, "k_sweep"),
+    (_swept, lambda st: st.icd(1, 1), 3, "k_sweep"),
+    (_built, lambda st: st.cost(), 1, "k_data_cost"),
+    (_tomo, _admm, 5, "k_fwdproj")])
+def test_a_group_of_buffers_is_whole_or_absent(L, make, call, n, kernel):
+    """Whichever buffer fails: the call after it allocates the whole group and
+    no kernel has run without it."""
+    live0 = L.stub_live()
+    whole = make()
+    call(whole)
+    live = L.stub_live()
+    whole.close()
+    for after in range(n):
+        st = make()
+        L.stub_clear_log()
+        L.stub_fail_malloc(after)
+        for _ in range(2):                      # the second: still no memory
+            with pytest.raises(RuntimeError):
+                call(st)
+        assert not any(kernel in k[0] for k in hip_stub.launches(L))
+        L.stub_fail_malloc(-1)
+        call(st)
+        assert L.stub_live() == live
+        st.close()
+        assert L.stub_live() == live0
+
+
+def test_a_tile_whose_lists_failed_is_not_kept(L):
+    """Back at the tile of the last sweep after a failed one: its lists are
+    made again, not taken for there."""
+    st = _built()
+    st.icd(1, 1)
+    st.option("tile", 4)
+    L.stub_fail_malloc(0)
+    with pytest.raises(RuntimeError):
+        st.icd(1, 1)
+    st.option("tile", 16)
+    L.stub_clear_log()
+    with pytest.raises(RuntimeError):
+        st.icd(1, 1)
+    assert not hip_stub.launches(L)
+    L.stub_fail_malloc(-1)
+    st.icd(1, 1)
+    st.close()
