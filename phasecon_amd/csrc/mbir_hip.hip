@@ -307,7 +307,9 @@ __global__ __launch_bounds__(kFwdThreads) void k_fwdproj(
           }
           const int k = ok ? (int)t : 0;
           const double2 h = s_h[k];
-          const double v = ok ? h.x + (t - k) * h.y : 0.0;
+          double v = h.x + (t - k) * h.y;
+          ok = ok && v > 0.0;  // the A rule keeps positive responses only
+          v = ok ? v : 0.0;
           const float* xc = xf + (size_t)(ok ? u * ni + i : 0) * G.N_z;
           if (vec) {
 #pragma unroll

@@ -81,6 +81,37 @@ def test_projections_match_the_system_matrix(rows, cols, views, frames, mxy, mz,
     st.close()
 
 
+def test_entries_that_a_does_not_hold():
+    """A keeps positive responses only: where the response table is zero or
+    negative the projection adds nothing, not even of an infinite voxel."""
+    from phasecon_amd import lib
+    from phasecon_amd.mbir import Stage, _p
+    st = Stage(_scan(5, 40, 6, 2))
+    st.L.mbir_hip_destroy(st.h)
+    st.H[:, 20:30] = 0.0
+    st.H[:, 40:] = -np.abs(st.H[:, 40:]) - 0.1
+    h = C.c_void_p()
+    lib.check(st.L.mbir_hip_create(C.byref(h), C.byref(st.g), _p(st.H), _p(st.cos), _p(st.sin),
+                                   _p(st.frame_ptr), _p(st.frame_views), _p(st.y), _p(st.w), None,
+                                   _p(st.mask)), "mbir_hip_create")
+    st.h = h
+    print("response table with zeros and negative values", flush=True)
+    _check(st, 4)
+    x = np.random.default_rng(4).random(st.shape_x).astype(np.float32)
+    want, _ = _dense(st, x, st.y)
+    x[0, 2, 17, 22] = np.inf
+    first, val = st.get_amatrix()
+    ax = st.forward_project(x)
+    st.close()
+    c = 17 * st.g.N_x + 22
+    hit = np.zeros(st.shape_e, bool)
+    for s in range(st.frame_ptr[0], st.frame_ptr[1]):
+        for k in np.nonzero(val[c, s])[0]:
+            hit[st.frame_views[s], first[c, s] + k, 2] = True
+    assert np.isinf(ax[hit]).all() and hit.any()
+    assert np.abs(ax - want)[~hit].max() <= 1e-6 * np.abs(want).max()
+
+
 @pytest.mark.parametrize("factor", [1.7, 0.6])
 def test_other_response_tables(factor):
     """A response table over another width than the usual one (the window of
