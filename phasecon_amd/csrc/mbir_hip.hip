@@ -208,13 +208,14 @@ __global__ __launch_bounds__(256) void k_aquant(int ncol, int per_col, float* __
 
 // ----------------------------------------------------------- projection
 // out [t][x][y][z] := in [t][y][x][z], tiles of 16 x 16 columns and up to 32
-// slices (blockIdx.z: frame and slice chunk) through LDS.
+// slices (blockIdx.x: frame and slice chunk, which may be more than the other
+// grid axes hold) through LDS.
 __global__ __launch_bounds__(256) void k_swap_xy(int Ny, int Nx, int Nz, int nzc,
                                                  const float* __restrict__ in,
                                                  float* __restrict__ out) {
   __shared__ float s[256 * 33];
-  const int f = blockIdx.z / nzc, z0 = (blockIdx.z - f * nzc) * 32, nz = min(32, Nz - z0);
-  const int x0 = blockIdx.x * 16, y0 = blockIdx.y * 16;
+  const int f = blockIdx.x / nzc, z0 = (blockIdx.x - f * nzc) * 32, nz = min(32, Nz - z0);
+  const int x0 = blockIdx.z * 16, y0 = blockIdx.y * 16;
   const size_t vol = (size_t)Ny * Nx * Nz;
   for (int i = threadIdx.x; i < 256 * nz; i += 256) {
     const int col = i / nz, z = i - col * nz, yy = y0 + (col >> 4), xx = x0 + (col & 15);
@@ -2196,8 +2197,8 @@ __global__ __launch_bounds__(kWave) void k_subst(SwGeom G, float alpha, int n,
   if (act && sub == 0) out[i] = substitute(alpha, v, th1[i], th2[i], num, den);
 }
 
-// A^T v: a workgroup takes 256 columns of one frame, a thread one of them and
-// kZ slices (blockIdx.z), whose sums it keeps in registers (z_overlap rows
+// A^T v: a workgroup takes 256 columns of one frame (blockIdx.x: frame and
+// block of columns), a thread one of them and kZ slices (blockIdx.y), whose sums it keeps in registers (z_overlap rows
 // folded into z); consecutive threads take consecutive columns, which read
 // neighbouring detector rows.  The columns' A goes through LDS, `sc` view
 // slots at a time, read as each column's contiguous run: a lane reading its
@@ -2215,8 +2216,8 @@ __global__ __launch_bounds__(256) void k_backproj(DevGeom G, int sc,
   extern __shared__ __align__(16) float smem[];
   float* s_a = smem;                                          // [sc W][257]
   int* s_f = reinterpret_cast<int*>(smem + sc * G.W * 257);   // [sc][257]
-  const int ncol = G.N_x * G.N_y, c0 = blockIdx.x * 256, c = c0 + threadIdx.x;
-  const int f = blockIdx.y, z0 = blockIdx.z * kZ;
+  const int ncol = G.N_x * G.N_y, ncb = (ncol + 255) / 256, f = blockIdx.x / ncb;
+  const int c0 = (blockIdx.x - f * ncb) * 256, c = c0 + threadIdx.x, z0 = blockIdx.y * kZ;
   const int s0 = frame_ptr[f], s1 = frame_ptr[f + 1], nc = min(256, ncol - c0);
   const bool vec = G.zo == 1 && (G.N_t & 3) == 0 && (G.N_z & 3) == 0 && z0 + kZ <= G.N_z;
   float acc[kZ];
@@ -2846,7 +2847,7 @@ int run_fwdproj(mbir_hip_ctx* c, int mode, const float* x, float* out,
   if (!c->d_xt && dev_alloc(&c->d_xt, c->nvox)) return -1;
   if (ev_begin(c, mode == 1 ? MBIR_K_COST : MBIR_K_FWDPROJ)) return -1;
   const int nzc = (g.N_z + 31) / 32;
-  hipLaunchKernelGGL(k_swap_xy, dim3((g.N_x + 15) / 16, (g.N_y + 15) / 16, g.N_time * nzc),
+  hipLaunchKernelGGL(k_swap_xy, dim3(g.N_time * nzc, (g.N_y + 15) / 16, (g.N_x + 15) / 16),
                      dim3(256), 0, c->stream, g.N_y, g.N_x, g.N_z, nzc, x, c->d_xt);
   const size_t lds = sizeof(double) * (kFwdThreads / 2) * q.kz;
   const auto go = [&](auto kernel) {
@@ -2875,7 +2876,7 @@ void launch_sweep(mbir_hip_ctx* c, const SweepArgs& A, unsigned nwg, size_t lds)
 // chunk of slices reads the stored A again).
 void launch_backproj(mbir_hip_ctx* c, const float* v, float* out) {
   const int kz = c->g.N_z <= 8 ? 8 : 32;
-  const dim3 grid((unsigned)((c->ncol + 255) / 256), (unsigned)c->g.N_time,
+  const dim3 grid((unsigned)((c->ncol + 255) / 256) * (unsigned)c->g.N_time,
                   (unsigned)((c->g.N_z + kz - 1) / kz));
   // 32 KiB of A at a time (W = 33: one slot, 35 KiB)
   const int sc = std::max(1, 32 / (1 + c->G.W));

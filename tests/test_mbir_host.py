@@ -1,5 +1,6 @@
 """The MBIR library's host side against a stand-in for the HIP runtime
-(hip_stub.py): what a failed allocation leaves behind."""
+(hip_stub.py): what a failed allocation leaves behind, and the grids of
+launches over many frames."""
 import os
 
 import numpy as np
@@ -109,3 +110,23 @@ def test_a_tile_whose_lists_failed_is_not_kept(L):
     L.stub_fail_malloc(-1)
     st.icd(1, 1)
     st.close()
+
+
+def test_grids_of_many_frames(L):
+    """Frames beyond what a grid's second and third axis hold (65535): every
+    launch of the projections puts them on the first."""
+    from phasecon_amd.mbir import Stage
+    from phasecon_amd.synth import geometry_scan
+    n = 66000
+    s = geometry_scan(1, 16, n)
+    s["recon_num"], s["recon_times"] = n, np.arange(n + 1).astype(np.float32)
+    st = Stage(s)
+    st.build_amatrix()
+    st.init_error()
+    st.backproject(np.zeros(st.shape_e, np.float32))
+    st.close()
+    runs = hip_stub.launches(L)
+    assert {k for k in ("k_swap_xy", "k_fwdproj", "k_backproj") if any(k in r[0] for r in runs)} \
+        == {"k_swap_xy", "k_fwdproj", "k_backproj"}
+    for name, x, y, z, threads in runs:
+        assert y <= 65535 and z <= 65535 and x * threads < 1 << 32, name
