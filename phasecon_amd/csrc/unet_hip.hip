@@ -110,6 +110,7 @@ struct ConvArgs {
   int cin_pad, cout, nt, relu;
   int lfx, lty, ltz;  // a workgroup's output tile: 16 fx x ty x tz voxels (log2)
   int ntx, ntz;       // tiles along x and z
+  int by, bz;         // first tile of the launch along y and along (volume, z)
 };
 
 // Channels of the input staged at once: all of up to 32, else 32, or 24 where
@@ -141,10 +142,11 @@ __device__ __forceinline__ uint4 conv_load(const ConvIn& I, int n, int z, int y,
 // workgroup stages its output tile's input with a one-voxel halo (zeros
 // outside the volume) in LDS once per channel chunk; its four wavefronts take
 // MV fragments of 16 voxels each (along x) and the NT output channel tiles of
-// 16 from blockIdx.y on.  One step multiplies 4 groups of 8 input channels of
-// one tap each (a lane's k group lane / 16) by weights that k_pack laid out
-// in fragment order (1 KiB per step and channel tile): one LDS read of 16
-// bytes per voxel fragment and no bounds test.  Weights are the A operand, so
+// 16 of its split (blockIdx.x counts splits, then tiles along x).  One step
+// multiplies 4 groups of 8 input channels of one tap each (a lane's k group
+// lane / 16) by weights that k_pack laid out in fragment order (1 KiB per step
+// and channel tile): one LDS read of 16 bytes per voxel fragment and no bounds
+// test.  Weights are the A operand, so
 // a lane ends with 4 consecutive channels of one voxel.
 // Bound by instruction issue around the MFMAs: staging, and at NT = 1 the LDS
 // reads (1 KiB per MFMA).  Reading the fragments from global memory, with the
@@ -164,9 +166,10 @@ __global__ __launch_bounds__(256) void k_conv(ConvArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int m = lane & 15, kg = lane >> 4;
   const int fx = 1 << a.lfx, HX = 16 * fx + 2, HY = (1 << a.lty) + 2, HZ = (1 << a.ltz) + 2;
-  const int split = blockIdx.x / a.ntx, n = blockIdx.z / a.ntz;
-  const int x0 = (blockIdx.x - split * a.ntx) * 16 * fx, y0 = blockIdx.y << a.lty;
-  const int z0 = (blockIdx.z - n * a.ntz) << a.ltz;
+  const unsigned bz = blockIdx.z + a.bz;
+  const int split = blockIdx.x / a.ntx, n = bz / a.ntz;
+  const int x0 = (blockIdx.x - split * a.ntx) * 16 * fx, y0 = (blockIdx.y + a.by) << a.lty;
+  const int z0 = (bz - n * a.ntz) << a.ltz;
   const int t0 = split * NT;
   int fb[MV];  // staged voxel index of the fragment's tap (-1, -1, -1)
 #pragma unroll
@@ -850,14 +853,20 @@ int launch_conv(hipStream_t s, const ConvIn& in, const u16* w, int cin_pad, int 
   if (V >= (1LL << 31)) return fail("too many voxels");
   const size_t lds = (size_t)((16 << a.lfx) + 2) * ((1 << a.lty) + 2) * ((1 << a.ltz) + 2) *
                      (conv_chunk(cin_pad) / 8) * 16;
-  const dim3 g((unsigned)a.ntx * (nt / NT), (unsigned)nty, (unsigned)a.ntz * N);
-  if (g.y > 65535 || g.z > 65535) return fail("volume too large");
-  switch (NT) {
-    case 1: conv_kernel<1>(s, a, mv, g, lds); break;
-    case 2: conv_kernel<2>(s, a, mv, g, lds); break;
-    case 3: conv_kernel<3>(s, a, mv, g, lds); break;
-    default: conv_kernel<4>(s, a, mv, g, lds); break;
-  }
+  // the y and z axes of a grid hold 65535 blocks: further tiles and volumes
+  // are launches of their own (one axis for all of them cost 1.3 % in divisions)
+  const int kAxis = 65535, ntnz = a.ntz * N;
+  for (a.bz = 0; a.bz < ntnz; a.bz += kAxis)
+    for (a.by = 0; a.by < nty; a.by += kAxis) {
+      const dim3 g((unsigned)a.ntx * (nt / NT), (unsigned)std::min(kAxis, nty - a.by),
+                   (unsigned)std::min(kAxis, ntnz - a.bz));
+      switch (NT) {
+        case 1: conv_kernel<1>(s, a, mv, g, lds); break;
+        case 2: conv_kernel<2>(s, a, mv, g, lds); break;
+        case 3: conv_kernel<3>(s, a, mv, g, lds); break;
+        default: conv_kernel<4>(s, a, mv, g, lds); break;
+      }
+    }
   HIP_OK(hipGetLastError());
   return 0;
 }

@@ -65,3 +65,17 @@ def test_network_with_chunked_channels(c, in_ch, shape):
     _, _, oy = U.unet_forward_backward(p32, x, t, c, bf16_storage=True)
     # the tolerance of test_unet_gradients_match_oracle (BF16 storage points)
     assert np.max(np.abs(y - oy)) <= 1e-2 * np.max(np.abs(oy))
+
+
+def test_more_volumes_than_a_grid_axis_holds():
+    """66000 volumes (a grid's second and third axis hold 65535), each equal
+    to one of three: the output of every one is that of its like in a small
+    batch.  The order of a voxel's sums does not depend on the batch."""
+    from phasecon_amd.warmstart import UNet
+    net = UNet(channels=8, seed=3)
+    x = np.random.default_rng(8).random((3, 4, 4, 64)).astype(np.float32)
+    print("66000 volumes of 4x4x64", flush=True)
+    want = net.forward(x)
+    y = net.forward(np.tile(x, (22000, 1, 1, 1))).reshape(22000, 3, 4, 4, 64)
+    net.close()
+    assert np.array_equal(y, np.broadcast_to(want, y.shape))

@@ -1,5 +1,6 @@
 """The network's host side against a stand-in for the HIP runtime
-(hip_stub.py): what a failed allocation leaves behind."""
+(hip_stub.py): what a failed allocation leaves behind, and the grids of
+launches over many volumes."""
 import os
 
 import numpy as np
@@ -40,3 +41,19 @@ def test_a_shape_whose_buffers_failed_is_not_kept(L, after):
     net.forward(small)
     net.close()
     assert L.stub_live() == live0
+
+
+@pytest.mark.parametrize("shape", [(66000, 4, 4, 64), (1, 4, 70000 * 8, 64)])
+def test_grids_of_many_tiles(L, shape):
+    """Volumes, and tiles along y, beyond what a grid's second and third axis
+    hold (65535)."""
+    from phasecon_amd.warmstart import UNet
+    net = UNet(channels=8)
+    x = np.zeros(shape, np.float32)
+    L.stub_clear_log()
+    net.forward(x)
+    net.close()
+    runs = hip_stub.launches(L)
+    assert sum("k_conv" in r[0] for r in runs) > 11
+    for name, gx, gy, gz, threads in runs:
+        assert gy <= 65535 and gz <= 65535 and gx * threads < 1 << 32, name
