@@ -835,19 +835,19 @@ int launch_conv(hipStream_t s, const ConvIn& in, const u16* w, int cin_pad, int 
     return fail("channel strides and offsets must be multiples of 8");
   if (out && (out->cs % 4 || out->co % 4))
     return fail("output channel strides and offsets must be multiples of 4");
-  if (nt != 1 && nt != 2 && nt != 3 && nt != 4 && nt != 6 && nt != 8)
-    return fail("unsupported channel count");
-  // 4 voxel fragments and up to 4 channel tiles per wavefront (64
-  // accumulator VGPRs; 8 fragments measured slower, 2.54 against 2.45 ms for
-  // the layers of 16 volumes of 8x256x256); fewer fragments, then fewer channel tiles, until the
-  // launch has two workgroups per CU
-  int NT = nt <= 4 ? nt : nt / 2, mv = 4, nty = 0;
+  // 4 voxel fragments and up to 4 channel tiles (a divisor of their number)
+  // per wavefront: 64 accumulator VGPRs (8 fragments measured slower, 2.54
+  // against 2.45 ms for the layers of 16 volumes of 8x256x256); fewer
+  // fragments, then fewer channel tiles, until the launch has two workgroups
+  // per CU
+  int NT = 4, mv = 4, nty = 0;
+  while (nt % NT) --NT;
   long long wgs = conv_tile(a, mv, &nty) * (nt / NT);
   while (wgs < 512 && (mv > 1 || NT > 1)) {
     if (mv > 1)
       mv /= 2;
     else
-      NT = NT % 2 ? 1 : NT / 2;
+      NT = NT % 2 ? 1 : NT / 2;  // still a divisor
     wgs = conv_tile(a, mv, &nty) * (nt / NT);
   }
   if (V >= (1LL << 31)) return fail("too many voxels");
