@@ -1196,8 +1196,23 @@ std::vector<float2> twiddles(int n) {
   return t;
 }
 
-// An event pair of the transforms' timing; collect_events sums them.
+// Sums the transforms' recorded times; waits for the stream.
+int collect_events(pcmbir_hip_ctx* c) {
+  HIP_OK(hipStreamSynchronize(c->stream));
+  for (size_t i = 0; i < c->ev_used; ++i) {
+    float m = 0.f;
+    HIP_OK(hipEventElapsedTime(&m, c->ev[i].first, c->ev[i].second));
+    c->fft_ms += m;
+  }
+  c->ev_used = 0;
+  return 0;
+}
+
+// An event pair of the transforms' timing.  The pairs are used again from
+// kMaxEvents on: one wait per so many, however long a descent runs.
+constexpr size_t kMaxEvents = 256;
 int fft_begin(pcmbir_hip_ctx* c) {
+  if (c->ev_used == kMaxEvents && collect_events(c)) return -1;
   if (c->ev_used == c->ev.size()) {
     hipEvent_t a, b;
     HIP_OK(hipEventCreate(&a));
@@ -1259,17 +1274,6 @@ int filter_dev(pcmbir_hip_ctx* c, float2* buf, int nbatch, const float2* fac) {
 // Fresnel transform (herm = 0: H, 1: H^H) of nbatch views stored at buf.
 int fresnel_dev(pcmbir_hip_ctx* c, float2* buf, int nbatch, int herm) {
   return filter_dev(c, buf, nbatch, herm ? c->fac_hh : c->fac_h);
-}
-
-int collect_events(pcmbir_hip_ctx* c) {
-  HIP_OK(hipStreamSynchronize(c->stream));
-  for (size_t i = 0; i < c->ev_used; ++i) {
-    float m = 0.f;
-    HIP_OK(hipEventElapsedTime(&m, c->ev[i].first, c->ev[i].second));
-    c->fft_ms += m;
-  }
-  c->ev_used = 0;
-  return 0;
 }
 
 unsigned ew_blocks(long long n) {

@@ -1,5 +1,6 @@
 """The phase retrieval's host side against a stand-in for the HIP runtime
-(hip_stub.py): what a failed allocation leaves behind."""
+(hip_stub.py): what a failed allocation leaves behind, and what a long descent
+holds."""
 import os
 
 import numpy as np
@@ -48,3 +49,18 @@ def test_a_group_of_buffers_is_whole_or_absent(L, call, n):
         assert L.stub_live() == live + n
         pr.close()
         assert L.stub_live() == live0
+
+
+@pytest.mark.parametrize("fft_reg", [0, 1])
+@pytest.mark.parametrize("thresh", [0.0, 1e-9])
+def test_a_long_descent_holds_no_more_events(L, fft_reg, thresh):
+    """The transforms' event pairs do not grow with the iterations."""
+    pr = _context()
+    pr.option("fft_reg", fft_reg)
+    _problem(pr)
+    pr.sd_run(1000, thresh)
+    held = L.stub_live_events()
+    pr.sd_run(2000, thresh)
+    assert L.stub_live_events() == held
+    pr.close()
+    assert L.stub_live_events() == 0
