@@ -1,7 +1,8 @@
 """The MBIR library's host side against a stand-in for the HIP runtime
-(hip_stub.py): what a failed allocation leaves behind, and the grids of
-launches over many frames."""
+(hip_stub.py): what a failed allocation leaves behind, the grids of launches
+over many frames, and the pinned memory of large copies."""
 import os
+import threading
 
 import numpy as np
 import pytest
@@ -130,3 +131,46 @@ def test_grids_of_many_frames(L):
         == {"k_swap_xy", "k_fwdproj", "k_backproj"}
     for name, x, y, z, threads in runs:
         assert y <= 65535 and z <= 65535 and x * threads < 1 << 32, name
+
+
+def _large():
+    from phasecon_amd.mbir import Stage
+    from phasecon_amd.synth import geometry_scan
+    return Stage(geometry_scan(33, 256, 2))     # an object of 8.25 MiB
+
+
+def _round_trip(st, seed):
+    x = np.random.default_rng(seed).random(st.shape_x, np.float32)
+    st.set_object(x)
+    return np.array_equal(st.get_object(), x)
+
+
+def test_contexts_share_the_pinned_slots(L):
+    """Contexts one after another share one set of slots, concurrent copies pin
+    at most four, and the last context gives them back; without pinned memory a
+    copy goes without."""
+    pins, live, events = L.stub_pins(), L.stub_live_pins(), L.stub_live_events()
+    sts = [_large() for _ in range(3)]
+    L.stub_fail_pin(1)
+    assert _round_trip(sts[0], 0)
+    L.stub_fail_pin(0)
+    assert L.stub_pins() == pins
+    assert all(_round_trip(st, i) for i, st in enumerate(sts))
+    assert L.stub_pins() == pins + 1 and L.stub_live_pins() == live + 1
+    sts.pop().close()
+    assert _round_trip(sts[0], 5) and L.stub_pins() == pins + 1
+    for st in sts:
+        st.close()
+    assert L.stub_live_pins() == live and L.stub_live_events() == events
+    sts, ok = [_large() for _ in range(6)], []
+    th = [threading.Thread(target=lambda st=st: ok.append([_round_trip(st, i) for i in range(8)]))
+          for st in sts]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert ok == [[True] * 8] * 6
+    assert 1 <= L.stub_live_pins() - live <= 4
+    for st in sts:
+        st.close()
+    assert L.stub_live_pins() == live and L.stub_live_events() == events
