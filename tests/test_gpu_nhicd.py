@@ -48,8 +48,7 @@ def test_vsc_filter_matches_oracle(small4d_scan):
 
 
 @pytest.mark.parametrize("fraction", [0.25, 0.1])
-def test_nh_pass_visits_the_top_columns_of_each_tile(small4d_scan, fraction):
-    T = 8
+def test_nh_pass_visits_the_top_columns_of_each_tile(small4d_scan, fraction, T=8):
     st = _stage(small4d_scan, T)
     st.icd(3, 1, 23)
     mag0 = st.magnitudes()

@@ -67,12 +67,16 @@ def _check(st, seed):
 
 
 # detectors below, at and above a workgroup's bins (32 to 512); one to 40
-# slices: below, at and above the slice chunks; rows per slice 1, 2 and 3;
-# an off-centre axis, where columns miss the detector
+# slices; rows per slice 1, 2 and 3; an off-centre axis, where columns miss the
+# detector.  Few workgroups take 4 slices each, whatever there are; from 256 on
+# 8 or 16: the second line has both, below, at and above a chunk
 @pytest.mark.parametrize("rows,cols,views,frames,mxy,mz,rot", [
     (1, 16, 7, 1, 1, 1, None), (3, 32, 5, 2, 1, 1, None), (8, 66, 9, 3, 1, 1, 20.0),
     (10, 64, 4, 1, 2, 2, None), (9, 60, 6, 2, 3, 3, None), (24, 48, 5, 2, 4, 1, 30.5),
-    (40, 34, 3, 1, 1, 1, None), (4, 520, 3, 1, 1, 1, None), (17, 130, 2, 2, 1, 1, None)])
+    (40, 34, 3, 1, 1, 1, None), (4, 520, 3, 1, 1, 1, None), (17, 130, 2, 2, 1, 1, None),
+    (7, 20, 130, 2, 1, 1, None), (8, 20, 130, 2, 1, 1, 7.5), (10, 20, 70, 2, 1, 1, None),
+    (13, 24, 130, 2, 1, 1, None), (16, 24, 130, 2, 2, 1, None), (20, 20, 65, 2, 1, 1, 11.0),
+    (34, 24, 130, 2, 1, 2, None)])
 def test_projections_match_the_system_matrix(rows, cols, views, frames, mxy, mz, rot):
     from phasecon_amd.mbir import Stage
     print(f"rows {rows}, cols {cols}, views {views} x {frames}, mult {mxy}/{mz}", flush=True)
@@ -112,13 +116,15 @@ def test_entries_that_a_does_not_hold():
     assert np.abs(ax - want)[~hit].max() <= 1e-6 * np.abs(want).max()
 
 
+# 4, 8 and 16 slices per workgroup
+@pytest.mark.parametrize("rows,cols,views", [(5, 40, 6), (7, 24, 130), (20, 24, 65)])
 @pytest.mark.parametrize("factor", [1.7, 0.6])
-def test_other_response_tables(factor):
+def test_other_response_tables(factor, rows, cols, views):
     """A response table over another width than the usual one (the window of
     the A rule then cuts it, or a bin meets more voxels of a line)."""
     from phasecon_amd import lib
     from phasecon_amd.mbir import Stage, _p
-    st = Stage(_scan(5, 40, 6, 2))
+    st = Stage(_scan(rows, cols, views, 2))
     st.L.mbir_hip_destroy(st.h)
     st.g.OffsetR *= factor
     h = C.c_void_p()
@@ -126,18 +132,20 @@ def test_other_response_tables(factor):
                                    _p(st.frame_ptr), _p(st.frame_views), _p(st.y), _p(st.w), None,
                                    _p(st.mask)), "mbir_hip_create")
     st.h = h
-    print(f"OffsetR x {factor}", flush=True)
+    print(f"OffsetR x {factor}, rows {rows}, cols {cols}, views {views} x 2", flush=True)
     _check(st, 3)
     st.close()
 
 
-@pytest.mark.parametrize("rows,cols,views", [(1, 32, 3), (20, 50, 4), (17, 400, 2)])
-def test_fbp_matches_numpy(rows, cols, views):
+# the last: more channels than the ramp filter stages
+@pytest.mark.parametrize("rows,cols,views,mxy", [
+    (1, 32, 3, 1), (20, 50, 4, 1), (17, 400, 2, 1), (2, 6208, 2, 16)])
+def test_fbp_matches_numpy(rows, cols, views, mxy):
     """A^T ramp(y) / K with the ramp as a dense FP64 matrix."""
     from phasecon_amd.mbir import Stage
     s = _scan(rows, cols, views, 1)
     s["projections"] = np.random.default_rng(1).random((views, rows, cols)).astype(np.float32)
-    st = Stage(s)
+    st = Stage(s, mult_xy=mxy)
     st.build_amatrix()
     print(f"fbp {rows}x{cols}, {views} views", flush=True)
     out = st.fbp()

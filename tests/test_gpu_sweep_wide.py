@@ -4,9 +4,14 @@ restatement of its schedule, as test_gpu_sweep_order.py does for the
 benchmark's shapes and with the same tolerance: one launch per tile colour
 and frame parity, so the sweep is the oracle's sequential ICD.
 
-The last test has launches of more workgroups than the chip has CUs, where
-the sinogram side takes two wavefronts and several tiles of a frame run at
-once: the maintained error sinogram stays y - A x and the cost falls.
+Launches of more workgroups than the chip has CUs give the sinogram side two
+wavefronts: with several hundred frames of one tile per colour they are just
+as deterministic; with several tiles of a frame at once (the last test) the
+maintained error sinogram stays y - A x and the cost falls.
+
+Non-homogeneous passes rank a tile's columns with all of a workgroup's
+threads, 192 or 320 here: test_gpu_nhicd.py's test on such geometries, with
+tiles of fewer and of more columns than threads.
 
 Shapes: row counts that are and are not powers of two and above one
 wavefront, view counts at both sides of a load batch and not a multiple of
@@ -25,16 +30,17 @@ pytestmark = pytest.mark.gpu
     (24, 32, 7), (24, 32, 29),    # 24 rows: 2 groups of 24 lanes
     (12, 32, 20), (34, 16, 17),   # 4 groups of 12, one group of 34
     (80, 16, 11)])                # rows above one wavefront
-def test_wide_sweep_matches_oracle_schedule(rows, cols, views):
+def test_wide_sweep_matches_oracle_schedule(rows, cols, views, frames=1):
     from oracle.oracle import Oracle
     from phasecon_amd.mbir import Stage
     from phasecon_amd.synth import make_scan
-    scan = make_scan("tall3d", seed=1, rows=rows, cols=cols, views=views)
+    scan = make_scan("tall3d", seed=1, rows=rows, cols=cols, views=views * frames, frames=frames)
     o = Oracle(scan)
     T = cols // 2
-    print(f"rows {rows}, cols {cols}, views {views}", flush=True)
+    print(f"rows {rows}, cols {cols}, views {views} x {frames}", flush=True)
     x0 = _start(o, 20, False)
     st = Stage(scan, tile=T, alpha=1.5)
+    st.option("pair_parities", 0)  # the launch order the oracle's model follows
     st.set_object(x0.astype(np.float32))
     st.build_amatrix()
     st.init_error()
@@ -52,6 +58,22 @@ def test_wide_sweep_matches_oracle_schedule(rows, cols, views):
     assert moved > 100 * TOL
     assert dx < TOL
     assert de < TOL
+
+
+# 260 workgroups in each launch
+@pytest.mark.parametrize("rows,views", [(3, 3), (5, 18), (24, 7)])
+def test_wide_sweep_of_many_frames_matches_oracle_schedule(rows, views):
+    test_wide_sweep_matches_oracle_schedule(rows, 12, views, 520)
+
+
+# four wavefronts (tile 8, 16: 64 and 256 columns, 320 threads), then two
+# (70 frames of 4 tiles per colour: 280 workgroups of 192 threads)
+@pytest.mark.parametrize("T,frames", [(8, 4), (16, 4), (16, 140)])
+def test_nh_pass_of_a_wide_sweep(T, frames):
+    from phasecon_amd.synth import make_scan
+    from test_gpu_nhicd import test_nh_pass_visits_the_top_columns_of_each_tile as check
+    print(f"tile {T}, {frames} frames", flush=True)
+    check(make_scan("tall3d", seed=2, rows=3, cols=64, views=7 * frames, frames=frames), 0.3, T)
 
 
 @pytest.mark.parametrize("rows,views", [(8, 20 * 16), (12, 7 * 16)])
