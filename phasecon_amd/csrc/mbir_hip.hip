@@ -14,11 +14,11 @@
 //   k_amatrix     A build, FP64 arithmetic identical to the reference rule
 //   k_fwdproj     A x per view gathered per detector bin in FP64, A recomputed
 //                 on the fly
-//   k_sweep       the parallel ICD: one wavefront per (tile, frame) walks the
+//   k_sweep       the parallel ICD: a workgroup per (tile, frame) walks the
 //                 tile's voxel columns in a seeded random order; theta1/theta2
-//                 reduced over the column's sparse footprint across the
-//                 wavefront, qGGMRF surrogate from an LDS-staged 3x3xN_z (+t+-1)
-//                 neighbourhood, error sinogram updated with atomics
+//                 reduced over the column's sparse footprint by 1, 2 or 4
+//                 wavefronts, qGGMRF surrogate from an LDS-staged 3x3xN_z (+t+-1)
+//                 neighbourhood by one, error sinogram updated with atomics
 //   k_prior_cost  FP64 prior term, k_data_cost FP64 data term
 //   k_backproj    A^T v, k_thetas / k_subst unit-test entry kernels
 #include <hip/hip_runtime.h>
@@ -236,9 +236,10 @@ __global__ __launch_bounds__(256) void k_swap_xy(int Ny, int Nx, int Nz, int nzc
 // response at |r - bin centre|, which vanishes from 64 OffsetR on.  For
 // 64 OffsetR = delta_xy / sqrt 2 + delta_r / 2 (kWindow = false) that lies
 // inside the A rule's window of W bins for every mult_xy, so the window tests
-// of amatrix_visit never cut it; other geometries run them (kWindow).  Along the image axis on which r changes faster
-// (|a| >= delta_xy / sqrt 2 per voxel), a bin then meets at most 4 voxels of a
-// line (kFwdCand, taken together).  A thread takes one bin and every G-th line, and sums kZ voxel
+// of amatrix_visit never cut it; other geometries run them (kWindow).  Along
+// the image axis on which r changes faster (|a| >= delta_xy / sqrt 2 per
+// voxel), a bin then meets at most 4 voxels of a line (kFwdCand, taken
+// together).  A thread takes one bin and every G-th line, and sums kZ voxel
 // slices in FP64 registers; the G threads of a bin meet in LDS (the same
 // order on every call).  Then e = y - A x - d (mode 0), the FP64 data cost of
 // y - A x - d (mode 1), or A x itself (mode 2).
@@ -551,12 +552,19 @@ __device__ __forceinline__ float substitute(float alpha, float V, float th1, flo
 
 // theta's reads of the shared error sinogram: workgroup-scope loads, which
 // skip the CU's L1 and are served by the XCD's L2.  An L2 copy of a line may
-// predate atomics performed since (by other XCDs' tiles, or at the memory
-// side), so theta can miss recent updates of concurrent tiles -- the
-// asynchronous staleness the parallel ICD already has, bounded by one launch
-// (a launch starts from coherent caches).  The sinogram itself stays exact:
-// every update is an agent-scope atomic.  Agent-scope loads (which refetch
-// past the L2) cost 10 % more time per launch for the same convergence.
+// predate atomics that other XCDs' tiles have sent since, so theta can miss
+// recent updates of concurrent tiles -- the asynchronous staleness the
+// parallel ICD already has, bounded by one launch (a launch starts from
+// coherent caches).  The sinogram itself stays exact: every update is an
+// agent-scope atomic.  Agent-scope loads (which refetch past the L2) cost 10 %
+// more time per launch for the same convergence.
+// A workgroup's own updates it does see, in order: both are atomic accesses,
+// and __syncthreads is a release and an acquire at workgroup scope, so a load
+// before it holds nothing of an update sent after it, by whichever wavefront,
+// and a load after it all of one sent before it.  On this target that takes no
+// wait on the accesses in flight, since the wavefronts of a workgroup share
+// their CU's path to memory, which keeps their order (threadgroup split mode,
+// which would let them sit on two CUs, is off unless compiled for).
 __device__ __forceinline__ float e_load(const float* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
@@ -784,9 +792,9 @@ struct Lanes {
 // generalized-Huber weight included) by nw wavefronts, wavefront wv taking
 // the view slots (j nw + wv) groups + g, j = 0, 1, ...: its share of every
 // row's sums lands in row1 / row2.  Each lane issues the e/w loads of a batch
-// of its slots back to back, then accumulates; entries with a = 0 load an
-// address of their own batch's first element and are not used, so that no
-// branch splits the batch.
+// of its slots back to back, then accumulates; entries with a = 0 load the
+// sinogram's first element and are not used, so that no branch splits the
+// batch.
 template <int kW>
 __device__ __forceinline__ void col_thetas(const SwGeom& G, const ColumnArgs& A, const Win& win,
                                            int nv, int wv, int nw, float* row1, float* row2) {
@@ -843,7 +851,10 @@ __device__ __forceinline__ void col_thetas(const SwGeom& G, const ColumnArgs& A,
 // a lane's row in SB slots, N_t <= 64 and a power of two): the e/w loads of
 // the next column go out while the current column is solved, and are
 // consumed after it, corrected for the current column's own error update,
-// which reaches the shared sinogram only after them.
+// which is sent only after them: by the same wavefront once it has consumed
+// them, or by the prior wavefront after the barrier that follows them (their
+// order: e_load).  The update before that one was sent before the barrier that
+// precedes them, so they hold it.
 template <int kW>
 struct ThetaLoads {
   static constexpr int SB = kW <= 5 ? 2 : 1;
@@ -876,8 +887,8 @@ __device__ __forceinline__ void theta_issue(const SwGeom& G, const ColumnArgs& A
 
 // theta1/theta2 per row from loads issued by theta_issue on window `win`,
 // first subtracting the previous column's own update (window `wprev`, voxel
-// changes dxp; has_prev = 0 for the first column), as the sinogram held no
-// part of it when the loads went out.
+// changes dxp; has_prev = 0 for the first column), of which the loads hold
+// nothing (ThetaLoads).
 template <int kW>
 __device__ __forceinline__ void theta_finish(const SwGeom& G, const Win& win, const Win& wprev,
                                              bool has_prev, const float* dxp, int lognt,
@@ -1247,13 +1258,14 @@ constexpr int kNhMax = 256;       // tile columns a non-homogeneous pass can ran
 // wavefront's loads complete in order behind its own atomics) where W = 3 or
 // the launch is small (SweepArgs::prior_sends); measured against the
 // sinogram wavefront sending them, ms per launch: 32x32x4 0.206 -> 0.168,
-// 256x256x8 paired tile 8 0.599 -> 0.585, tile 12 0.617 -> 0.553.  kNS = 2 or 4 elsewhere: the view slots are dealt over kNS
-// wavefronts, so that a column is still one load batch per lane (one memory
-// round trip) and not a chain of them; each wavefront sends the error update
-// of its own slots and then loads them for the next column, so a column sees
-// its own tile's updates without a correction.  Bound by that chain (update,
-// load, sum, solve), not by bandwidth: 150 columns x 24 rows at half
-// resolution, 29 views per frame, W = 5, tile 8: 1.191 -> 0.418 ms per launch (6.5 us per column).
+// 256x256x8 paired tile 8 0.599 -> 0.585, tile 12 0.617 -> 0.553.
+// kNS = 2 or 4 elsewhere: the view slots are dealt over kNS wavefronts, so
+// that a column is still one load batch per lane (one memory round trip) and
+// not a chain of them; each wavefront sends the error update of its own slots
+// and then loads them for the next column, so a column sees its own tile's
+// updates without a correction.  Bound by that chain (update, load, sum,
+// solve), not by bandwidth: 150 columns x 24 rows at half resolution, 29 views
+// per frame, W = 5, tile 8: 1.191 -> 0.418 ms per launch (6.5 us per column).
 // kW = W, the A window width.
 // The small-frame pipelined variants with window widths up to 5 are compiled
 // for exactly four wavefronts per SIMD: at 128x128x4 with tile 4 a launch's
@@ -2835,6 +2847,9 @@ FwdPlan fwd_plan(const mbir_hip_geom& g) {
 int run_fwdproj(mbir_hip_ctx* c, int mode, const float* x, float* out,
                 const float* y = nullptr, double xscale = 1.0) {
   const mbir_hip_geom& g = c->g;
+  // the widest detectors the interface takes (14336 channels for A x, 7168 for
+  // e and the cost); the kernel's LDS does not depend on the width, but the
+  // ramp filter's table does (launch_ramp: 112 KiB at 14336)
   if ((size_t)g.N_r * (mode == 2 ? 4 : 8) > 56 * 1024)
     return fail("detector too wide for the projection");
   const FwdPlan q = fwd_plan(g);

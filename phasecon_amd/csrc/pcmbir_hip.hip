@@ -147,8 +147,7 @@ __host__ __device__ inline int col_tile(int logr, int logc) {
 
 // Per (view, tile of TC columns): forward FFT along rows, times fac
 // [rows][cols], inverse FFT along rows (of the views whose active flag is
-// set; NULL: all).  LDS rows are padded by one value
-// against bank conflicts.
+// set; NULL: all).  LDS rows are padded by one value against bank conflicts.
 __global__ __launch_bounds__(kThreads) void k_fresnel_cols(float2* __restrict__ data, int logr,
                                                            int logc,
                                                            const float2* __restrict__ twg,
@@ -570,7 +569,7 @@ __global__ __launch_bounds__(kThreads) void k_pr_cost(PrArgs P, double* __restri
 // away: H^H is linear, so the gradient's two Hermitian terms are one transform
 // of their difference, and H D w of the phase projection is that of the next
 // iteration's gradient.  Per pixel and iteration 240 bytes move instead of
-// 568: HBM-bound, 24 views of 512 x 512 0.87 -> 0.35 ms per iteration (4.3
+// 568: HBM-bound, 24 views of 512 x 512 0.87 -> 0.33 ms per iteration (4.6
 // TB/s over all its passes).
 enum RowStep {
   kRowsStart,     // D w -> forward
@@ -1239,7 +1238,8 @@ void cols_dev(pcmbir_hip_ctx* c, float2* buf, int nbatch, const float2* fac, con
     const unsigned threads = 1u << (ltc + c->logr - 3);
     const size_t lds = (sizeof(float2) << (ltc + c->logr)) + (sizeof(float2) << (c->logr - 1));
     hipLaunchKernelGGL(k_fresnel_cols_reg, dim3((unsigned)nbatch << (c->logc - ltc)),
-                       dim3(threads), lds, c->stream, buf, c->logr, c->logc, ltc, c->tw_r, fac, active);
+                       dim3(threads), lds, c->stream, buf, c->logr, c->logc, ltc, c->tw_r, fac,
+                       active);
   } else {
     const int tiles = c->cols / col_tile(c->logr, c->logc);
     hipLaunchKernelGGL(k_fresnel_cols, dim3((unsigned)(nbatch * tiles)), dim3(kThreads), 0,

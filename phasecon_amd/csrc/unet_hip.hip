@@ -12,9 +12,9 @@
 // [n][z][y][x][channel stride]; a layer reads / writes a channel range
 // (offset, count) of a buffer.  A decoder layer's input, the concatenation of
 // an up-sampled half-resolution buffer and a skip, is read from both places
-// and never written out (its gradient is).  Parameters, gradients and Adam moments: FP32, one buffer
-// each, per layer [cout][27][cin] (tap = (dz+1)*9 + (dy+1)*3 + (dx+1)) then
-// [cout]; BF16 copies of the weights in MFMA fragment order for the forward
+// and never written out (its gradient is).  Parameters, gradients and Adam
+// moments: FP32, one buffer each, per layer [cout][27][cin] (tap = (dz+1)*9 +
+// (dy+1)*3 + (dx+1)) then [cout]; BF16 copies of the weights in MFMA fragment order for the forward
 // GEMM and, with taps flipped and channels swapped, the backward-data GEMM.
 //
 // Kernels
@@ -22,8 +22,8 @@
 //                the tile's input with halo in LDS; forward (bias, ReLU) and
 //                backward-data (flipped weights)
 //   k_conv_dw    weight and bias gradient: 16 x 16 channels x 27 taps per
-//                workgroup, reduced over voxel rows with MFMA, FP32 atomics
-//                into the gradient
+//                workgroup, reduced over voxel rows with MFMA, FP32 sums per
+//                workgroup that k_dw_sum adds up in their order
 //   k_pool / k_pool_bwd, k_up_bwd, k_relu_bwd, k_mse, k_adam, k_pack
 //                elementwise / reduction helpers
 #include <hip/hip_runtime.h>
@@ -347,21 +347,23 @@ __device__ __forceinline__ void dw_put(char* dst, int st, uint4 v0, uint4 v1) {
 }
 
 // dW[co][tap][ci] = sum over voxels of g[v][co] in[v + d_tap][ci], and
-// db[co] = sum g[v][co], partial sums per workgroup: a workgroup takes 16 output channels (blockIdx.z),
-// 16 input channels (blockIdx.y) and `per` tiles of 8 output rows of 32
-// voxels; the MFMA's k runs over a row's 32 input voxels.  Per tile the input
-// rows with their y and z halo and three copies of the gradient rows, shifted
-// by -1, 0 and 1 voxels against them, go to LDS transposed (channel rows,
-// voxels contiguous), so that every fragment is one aligned 16-byte read and
-// the three x taps share the input fragment.  A wavefront takes two of the
-// rows and all 27 taps (108 accumulator VGPRs): 9 input and 3 gradient
-// fragments per 27 MFMAs.  The wavefronts' sums meet in LDS, the workgroups'
-// in k_dw_sum (1024 workgroups' atomics on one gradient took 160 of the
-// 225 us of a 16-to-16-channel layer over 262144 voxels).  Bound by the LDS traffic (staging and
-// fragments); gathering both operands voxel by voxel from global memory was
-// bound by its 16 scalar 2-byte loads per MFMA.  8 volumes of 8x64x64, 16 base
-// channels: the 11 layers 5.01 ms (and 0.24 ms for the bias sums) -> 0.24 ms;
-// 16 to 16 channels at full size 0.46 -> 0.019 ms.
+// db[co] = sum g[v][co], partial sums per workgroup: a workgroup takes 16
+// output channels (blockIdx.z), 16 input channels (blockIdx.y) and `per` tiles
+// of 8 output rows of 32 voxels; the MFMA's k runs over a row's 32 input
+// voxels.  Per tile the input rows with their y and z halo and three copies of
+// the gradient rows, shifted by -1, 0 and 1 voxels against them, go to LDS
+// transposed (channel rows, voxels contiguous), so that every fragment is one
+// aligned 16-byte read and the three x taps share the input fragment.  A
+// wavefront takes two of the rows and all 27 taps: 9 input and 3 gradient
+// fragments per 27 MFMAs, 112 accumulators with the bias's (AGPRs) beside 124
+// VGPRs and 32 bytes of scratch per lane, two wavefronts per SIMD.  The
+// wavefronts' sums meet in LDS, the workgroups' in k_dw_sum (1024 workgroups'
+// atomics on one gradient took 160 of the 225 us of a 16-to-16-channel layer
+// over 262144 voxels).  Bound by the LDS traffic (staging and fragments);
+// gathering both operands voxel by voxel from global memory was bound by its
+// 16 scalar 2-byte loads per MFMA.  8 volumes of 8x64x64, 16 base channels: the
+// 11 layers 5.01 ms (and 0.24 ms for the bias sums) -> 0.24 ms; 16 to 16
+// channels at full size 0.46 -> 0.019 ms.
 __global__ __launch_bounds__(256) void k_conv_dw(DwArgs a) {
   __shared__ uint4 s_i[16 * kDwSi];
   __shared__ uint4 s_g[3 * 16 * kDwSg];
@@ -440,7 +442,7 @@ __global__ __launch_bounds__(256) void k_conv_dw(DwArgs a) {
     }
   }
   // the four wavefronts' sums, in wavefront order (9 taps at a time fit the
-  // input rows' buffer), then the workgroup's into dw; a lane holds input
+  // input rows' buffer), then the workgroup's into part; a lane holds input
   // channel ci0 + m of output channels co0 + 4 kg + 0..3
   float* red = reinterpret_cast<float*>(s_i);  // [9 taps][4][64], 4 wavefronts of it in turn
 #pragma unroll
