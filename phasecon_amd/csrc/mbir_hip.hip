@@ -208,26 +208,29 @@ __global__ __launch_bounds__(256) void k_aquant(int ncol, int per_col, float* __
 
 // ----------------------------------------------------------- projection
 // out [t][x][y][z] := in [t][y][x][z], tiles of 16 x 16 columns and up to 32
-// slices (blockIdx.x: frame and slice chunk, which may be more than the other
-// grid axes hold) through LDS.
-__global__ __launch_bounds__(256) void k_swap_xy(int Ny, int Nx, int Nz, int nzc,
+// slices through LDS; n frames' slice chunks, which may be more than the grid's
+// z axis holds (65535).
+__global__ __launch_bounds__(256) void k_swap_xy(int Ny, int Nx, int Nz, int nzc, int n,
                                                  const float* __restrict__ in,
                                                  float* __restrict__ out) {
   __shared__ float s[256 * 33];
-  const int f = blockIdx.x / nzc, z0 = (blockIdx.x - f * nzc) * 32, nz = min(32, Nz - z0);
-  const int x0 = blockIdx.z * 16, y0 = blockIdx.y * 16;
+  const int x0 = blockIdx.x * 16, y0 = blockIdx.y * 16;
   const size_t vol = (size_t)Ny * Nx * Nz;
-  for (int i = threadIdx.x; i < 256 * nz; i += 256) {
-    const int col = i / nz, z = i - col * nz, yy = y0 + (col >> 4), xx = x0 + (col & 15);
-    if (yy < Ny && xx < Nx)
-      s[col * 33 + z] = in[f * vol + ((size_t)yy * Nx + xx) * Nz + z0 + z];
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < 256 * nz; i += 256) {
-    const int col = i / nz, z = i - col * nz, xx = x0 + (col >> 4), yy = y0 + (col & 15);
-    if (yy < Ny && xx < Nx)
-      out[f * vol + ((size_t)xx * Ny + yy) * Nz + z0 + z] =
-          s[((col & 15) * 16 + (col >> 4)) * 33 + z];
+  for (int fz = blockIdx.z; fz < n; fz += gridDim.z) {
+    const int f = fz / nzc, z0 = (fz - f * nzc) * 32, nz = min(32, Nz - z0);
+    if (fz >= (int)gridDim.z) __syncthreads();  // the last chunk has been read
+    for (int i = threadIdx.x; i < 256 * nz; i += 256) {
+      const int col = i / nz, z = i - col * nz, yy = y0 + (col >> 4), xx = x0 + (col & 15);
+      if (yy < Ny && xx < Nx)
+        s[col * 33 + z] = in[f * vol + ((size_t)yy * Nx + xx) * Nz + z0 + z];
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 256 * nz; i += 256) {
+      const int col = i / nz, z = i - col * nz, xx = x0 + (col >> 4), yy = y0 + (col & 15);
+      if (yy < Ny && xx < Nx)
+        out[f * vol + ((size_t)xx * Ny + yy) * Nz + z0 + z] =
+            s[((col & 15) * 16 + (col >> 4)) * 33 + z];
+    }
   }
 }
 
@@ -246,9 +249,9 @@ __global__ __launch_bounds__(256) void k_swap_xy(int Ny, int Nx, int Nz, int nzc
 // Bound by FP64 arithmetic and the loads of the voxel lines from L2; a
 // scatter with FP64 LDS atomics ran into their conflicts (voxels of a line
 // share bins) and formed each column's window once per chunk of rows.
-// 256 views of 256 bins x 8 rows, 256x256x8 voxels per frame: 0.893 ->
-// 0.181 ms (mode 2, FP32 atomics before: 1.604 ms); 360 views of 256 x 256,
-// 256^3 voxels: 18.5 -> 7.7 ms.
+// 256 views of 256 bins x 8 rows, 256x256x8 voxels per frame: 0.893 -> 0.174
+// ms and 0.032 for the exchange (mode 2, FP32 atomics before: 1.604 ms); 360
+// views of 256 x 256, 256^3 voxels: 18.5 -> 7.7 ms.
 // The lines run along y where that is the axis of faster r; those views read
 // xt, the object with x and y exchanged (k_swap_xy), so that neighbouring
 // bins always read neighbouring voxel columns.
@@ -263,7 +266,7 @@ __global__ __launch_bounds__(kFwdThreads) void k_fwdproj(
     const float* __restrict__ d, float* __restrict__ out,
     double* __restrict__ partial, double xscale) {
   extern __shared__ __align__(16) double s_acc[];  // [kFwdThreads / 2][kZ]
-  __shared__ double2 s_h[kRespBins];               // response and its step to the next entry
+  __shared__ double2 s_h[kRespBins + 1];  // response and its step to the next entry; past it 0
   const int p = blockIdx.x, z0 = blockIdx.y * kZ, nb = 1 << lognb;
   const int tid = threadIdx.x, j = blockIdx.z * nb + (tid & (nb - 1)), g = tid >> lognb;
   const int ng = kFwdThreads >> lognb;
@@ -271,6 +274,7 @@ __global__ __launch_bounds__(kFwdThreads) void k_fwdproj(
     const double h0 = H[(size_t)p * kNB + tid], h1 = H[(size_t)p * kNB + tid + 1];
     s_h[tid] = make_double2(h0, h1 - h0);
   }
+  if (tid == kRespBins) s_h[tid] = make_double2(0.0, 0.0);
   __syncthreads();
   double acc[kZ];
 #pragma unroll
@@ -300,18 +304,16 @@ __global__ __launch_bounds__(kFwdThreads) void k_fwdproj(
           if (q >= left) break;
           const int i = i0 + q;
           const double r = a * i + b, t = fabs(r - centre) * inv_off;
-          bool ok = i >= 0 && i < ni && t < (double)kRespBins;
+          const int k = min((int)t, kRespBins);
+          const double2 h = s_h[k];
+          const double v = h.x + (t - k) * h.y;
+          bool ok = (unsigned)i < (unsigned)ni && v > 0.0;  // A keeps positive responses only
           if (kWindow) {
             const double lo = r - G.delta_xy, hi = r + G.delta_xy;
             const int jlo = max(0, (int)floor((lo - G.R0) / G.delta_r));
             ok = ok && hi >= G.R0 && lo <= G.RMax && j >= jlo && j - jlo < G.W &&
                  j <= (int)floor((hi - G.R0) / G.delta_r);
           }
-          const int k = ok ? (int)t : 0;
-          const double2 h = s_h[k];
-          double v = h.x + (t - k) * h.y;
-          ok = ok && v > 0.0;  // the A rule keeps positive responses only
-          v = ok ? v : 0.0;
           const float* xc = xf + (size_t)(ok ? u * ni + i : 0) * G.N_z;
           if (vec) {
 #pragma unroll
@@ -2862,8 +2864,9 @@ int run_fwdproj(mbir_hip_ctx* c, int mode, const float* x, float* out,
   if (!c->d_xt && dev_alloc(&c->d_xt, c->nvox)) return -1;
   if (ev_begin(c, mode == 1 ? MBIR_K_COST : MBIR_K_FWDPROJ)) return -1;
   const int nzc = (g.N_z + 31) / 32;
-  hipLaunchKernelGGL(k_swap_xy, dim3(g.N_time * nzc, (g.N_y + 15) / 16, (g.N_x + 15) / 16),
-                     dim3(256), 0, c->stream, g.N_y, g.N_x, g.N_z, nzc, x, c->d_xt);
+  hipLaunchKernelGGL(
+      k_swap_xy, dim3((g.N_x + 15) / 16, (g.N_y + 15) / 16, std::min(65535, g.N_time * nzc)),
+      dim3(256), 0, c->stream, g.N_y, g.N_x, g.N_z, nzc, g.N_time * nzc, x, c->d_xt);
   const size_t lds = sizeof(double) * (kFwdThreads / 2) * q.kz;
   const auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, q.grid, dim3(kFwdThreads), lds, c->stream, c->G, mode, q.lognb,
