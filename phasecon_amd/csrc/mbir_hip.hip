@@ -2681,7 +2681,8 @@ struct mbir_hip_ctx {
   float *d_x = nullptr, *d_stage = nullptr, *d_stage2 = nullptr;
   uint8_t* d_mask = nullptr;  // update mask [N_y * N_x]
   float* d_ws = nullptr;      // warm-start sinogram scratch (allocated on first use)
-  float* d_xt = nullptr;      // object with x and y exchanged, for the projector (first use)
+  float* d_xt = nullptr;      // object with x and y exchanged, for A x (first use)
+  bool lines_y = false;       // a view's image lines run along y: it reads the exchanged object
   std::vector<float> offset;  // ring offset d [N_r][N_t] (host copy of d_d)
   // ring-offset windows (mode 3): per sinogram entry the windows covering it
   // and their weights, [off_cover_ptr[k], off_cover_ptr[k + 1])
@@ -2861,16 +2862,20 @@ int run_fwdproj(mbir_hip_ctx* c, int mode, const float* x, float* out,
                         fabs(g.delta_xy - g.mult_xy * g.delta_r) <= 1e-9 * g.delta_xy &&
                         fabs(g.RMax - g.R0 - g.N_r * g.delta_r) <= 1e-9 * g.delta_xy);
   if (mode == 1 && ensure_partial(c, (size_t)q.grid.x * q.grid.y * q.grid.z)) return -1;
-  if (!c->d_xt && dev_alloc(&c->d_xt, c->nvox)) return -1;
+  // the exchanged object, where a view reads it: in d_stage, which e and the
+  // cost leave free, so that only A x needs room for a second object
+  if (c->lines_y && mode == 2 && !c->d_xt && dev_alloc(&c->d_xt, c->nvox)) return -1;
+  float* const xt = mode == 2 ? c->d_xt : c->d_stage;
   if (ev_begin(c, mode == 1 ? MBIR_K_COST : MBIR_K_FWDPROJ)) return -1;
   const int nzc = (g.N_z + 31) / 32;
-  hipLaunchKernelGGL(
-      k_swap_xy, dim3((g.N_x + 15) / 16, (g.N_y + 15) / 16, std::min(65535, g.N_time * nzc)),
-      dim3(256), 0, c->stream, g.N_y, g.N_x, g.N_z, nzc, g.N_time * nzc, x, c->d_xt);
+  if (c->lines_y)
+    hipLaunchKernelGGL(
+        k_swap_xy, dim3((g.N_x + 15) / 16, (g.N_y + 15) / 16, std::min(65535, g.N_time * nzc)),
+        dim3(256), 0, c->stream, g.N_y, g.N_x, g.N_z, nzc, g.N_time * nzc, x, xt);
   const size_t lds = sizeof(double) * (kFwdThreads / 2) * q.kz;
   const auto go = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, q.grid, dim3(kFwdThreads), lds, c->stream, c->G, mode, q.lognb,
-                       c->d_H, c->d_cos, c->d_sin, c->d_view_frame, x, c->d_xt, y ? y : c->d_y,
+                       c->d_H, c->d_cos, c->d_sin, c->d_view_frame, x, xt, y ? y : c->d_y,
                        c->d_w, y ? nullptr : c->d_d, out, c->d_partial, xscale);
   };
   if (window)
@@ -2979,6 +2984,7 @@ int mbir_hip_create(mbir_hip_ctx** out, const mbir_hip_geom* g, const float* H,
         return fail("frame_views entry out of range");
       }
       view_frame[frame_views[s]] = f;
+      c->lines_y |= fabs(cosv[frame_views[s]]) < fabs(sinv[frame_views[s]]);  // as k_fwdproj
     }
   int rc = 0;
   int dev = 0, lds = 0;

@@ -85,6 +85,18 @@ def test_projections_match_the_system_matrix(rows, cols, views, frames, mxy, mz,
     st.close()
 
 
+# every view's image lines along x, along y
+@pytest.mark.parametrize("lo,hi", [(-0.78, 0.78), (0.79, 2.35)])
+def test_views_of_one_axis(lo, hi):
+    from phasecon_amd.mbir import Stage
+    s = _scan(6, 48, 5, 2)
+    s["angles"] = np.linspace(lo, hi, 10).astype(np.float32)
+    print(f"angles {lo} to {hi}", flush=True)
+    st = Stage(s)
+    _check(st, 9)
+    st.close()
+
+
 def test_entries_that_a_does_not_hold():
     """A keeps positive responses only: where the response table is zero or
     negative the projection adds nothing, not even of an infinite voxel."""

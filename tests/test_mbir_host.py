@@ -1,6 +1,7 @@
 """The MBIR library's host side against a stand-in for the HIP runtime
 (hip_stub.py): what a failed allocation leaves behind, the grids of launches
-over many frames, and the pinned memory of large copies."""
+over many frames, the pinned memory of large copies, and the projector's
+exchanged object."""
 import os
 import threading
 
@@ -174,3 +175,27 @@ def test_contexts_share_the_pinned_slots(L):
     for st in sts:
         st.close()
     assert L.stub_live_pins() == live and L.stub_live_events() == events
+
+
+def test_the_exchanged_object_takes_no_room_of_its_own(L):
+    """The error sinogram and the cost exchange x and y in the staging buffer;
+    A x alone allocates for it, and nothing is exchanged where no view's lines
+    run along y."""
+    from phasecon_amd.mbir import Stage
+    st = _built()
+    live = L.stub_live()
+    st.init_error()
+    assert L.stub_live() == live
+    assert any("k_swap_xy" in r[0] for r in hip_stub.launches(L))
+    st.forward_project(np.zeros(st.shape_x, np.float32))
+    assert L.stub_live() == live + 1
+    st.close()
+    s = _scan()
+    s["angles"] = np.linspace(-0.7, 0.7, 6).astype(np.float32)
+    st = Stage(s)
+    L.stub_clear_log()
+    st.init_error()
+    st.forward_project(np.zeros(st.shape_x, np.float32))
+    st.close()
+    runs = [r[0] for r in hip_stub.launches(L)]
+    assert any("k_fwdproj" in r for r in runs) and not any("k_swap_xy" in r for r in runs)
