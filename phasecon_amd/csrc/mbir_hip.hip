@@ -1252,8 +1252,8 @@ constexpr int kNhMax = 256;       // tile columns a non-homogeneous pass can ran
 //      the neighbours outside the column;
 //   2. the prior wavefront solves the z-parity halves (each voxel sees its
 //      z+-1 neighbours' new values).
-// kNS = 1, where a column's whole window is one load batch of one wavefront
-// (sweep_pipes): theta is pipelined -- the next column's loads go out during
+// kPipe, where a column's whole window is one load batch of one wavefront
+// (sweep_pipes; kNS = 1): theta is pipelined -- the next column's loads go out during
 // the solve, and are corrected for the column's own update, whose atomics
 // follow.  The prior wavefront sends those after its fixed terms (it waits
 // for no load, so their completion is on nobody's path: the sinogram
@@ -1261,11 +1261,12 @@ constexpr int kNhMax = 256;       // tile columns a non-homogeneous pass can ran
 // the launch is small (SweepArgs::prior_sends); measured against the
 // sinogram wavefront sending them, ms per launch: 32x32x4 0.206 -> 0.168,
 // 256x256x8 paired tile 8 0.599 -> 0.585, tile 12 0.617 -> 0.553.
-// kNS = 2 or 4 elsewhere: the view slots are dealt over kNS wavefronts, so
-// that a column is still one load batch per lane (one memory round trip) and
-// not a chain of them; each wavefront sends the error update of its own slots
-// and then loads them for the next column, so a column sees its own tile's
-// updates without a correction.  Bound by that chain (update, load, sum,
+// Elsewhere the view slots are dealt over kNS wavefronts, 2 or 4, so that a
+// column is still one load batch per lane (one memory round trip) and not a
+// chain of them, or left to one where a launch fills the chip without them
+// (sweep_waves); each wavefront sends the error update of its own slots and
+// then loads them for the next column, so a column sees its own tile's updates
+// without a correction.  Bound by that chain (update, load, sum,
 // solve), not by bandwidth: 150 columns x 24 rows at half resolution, 29 views
 // per frame, W = 5, tile 8: 1.191 -> 0.418 ms per launch (6.5 us per column).
 // kW = W, the A window width.
@@ -1275,10 +1276,10 @@ constexpr int kNhMax = 256;       // tile columns a non-homogeneous pass can ran
 // scheduler, free to use 128 VGPRs, keeps the pipelined loads in flight (left
 // to aim for five it takes 88 VGPRs and 0.672 instead of 0.600 ms per launch
 // at 256x256x8, tile 8, paired).
-template <int kW, bool kSmall, bool kHalf, int kNS>
+template <int kW, bool kSmall, bool kHalf, int kNS, bool kPipe>
 __global__ __launch_bounds__((kNS + 1) * kWave)
-__attribute__((amdgpu_waves_per_eu((kSmall && kW <= 5 && kNS == 1) ? 4 : 1,
-                                   (kSmall && kW <= 5 && kNS == 1) ? 4 : 8))) void
+__attribute__((amdgpu_waves_per_eu((kSmall && kW <= 5 && kPipe) ? 4 : 1,
+                                   (kSmall && kW <= 5 && kPipe) ? 4 : 8))) void
 k_sweep(SwGeom G, SweepArgs A) {
   constexpr int kThreads = (kNS + 1) * kWave;
   extern __shared__ __align__(16) float smem[];
@@ -1293,7 +1294,7 @@ k_sweep(SwGeom G, SweepArgs A) {
   // and each wavefront executes only its own loop's barriers.
   const int wv = kNS == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid) / kWave;
   const bool w0 = __builtin_amdgcn_readfirstlane(tid) < kNS * kWave;
-  const bool prior_sends = kNS == 1 && (kW == 3 || A.prior_sends != 0);
+  const bool prior_sends = kPipe && (kW == 3 || A.prior_sends != 0);
   const int wid_all = blockIdx.x;
   const int iter = A.iter_dev ? *A.iter_dev + A.iter : A.iter;
   load_prior(G, &s_prior);
@@ -1417,7 +1418,7 @@ k_sweep(SwGeom G, SweepArgs A) {
   SolveStats st;
   // Each wavefront runs its own loop over the columns; both loops pass the
   // same two workgroup barriers per column, so the phases stay aligned.
-  if (w0 && kNS == 1) {
+  if (w0 && kPipe) {
     const int lognt = __builtin_ctz((unsigned)G.N_t);
     ThetaLoads<kW> tl;
     // pipeline: the prefetch of column k+1 is in flight during column k's
@@ -2885,14 +2886,14 @@ int run_fwdproj(mbir_hip_ctx* c, int mode, const float* x, float* out,
   return ev_end(c, mode == 1 ? MBIR_K_COST : MBIR_K_FWDPROJ);
 }
 
-template <int kW, bool kSmall, int kNS>
+template <int kW, bool kSmall, int kNS, bool kPipe>
 void launch_sweep(mbir_hip_ctx* c, const SweepArgs& A, unsigned nwg, size_t lds) {
   if (c->afp16)
-    hipLaunchKernelGGL((k_sweep<kW, kSmall, true, kNS>), dim3(nwg), dim3((kNS + 1) * kWave), lds,
-                       c->stream, c->SG, A);
+    hipLaunchKernelGGL((k_sweep<kW, kSmall, true, kNS, kPipe>), dim3(nwg), dim3((kNS + 1) * kWave),
+                       lds, c->stream, c->SG, A);
   else
-    hipLaunchKernelGGL((k_sweep<kW, kSmall, false, kNS>), dim3(nwg), dim3((kNS + 1) * kWave), lds,
-                       c->stream, c->SG, A);
+    hipLaunchKernelGGL((k_sweep<kW, kSmall, false, kNS, kPipe>), dim3(nwg),
+                       dim3((kNS + 1) * kWave), lds, c->stream, c->SG, A);
 }
 
 // out := A^T v: slices per thread 8, or 32 where a column has more (each
@@ -3323,14 +3324,27 @@ bool sweep_pipes(const mbir_hip_ctx* c) {
          c->nvmax <= (c->G.W <= 5 ? 2 : 1) * (kWave / nt);
 }
 
+// Frames whose window one wavefront stages in 1 + 4 registers per lane.
+bool sweep_small(const mbir_hip_ctx* c) {
+  return c->nvmax <= kWave && c->nvmax * c->G.W <= 4 * kWave;
+}
+
 // Sinogram wavefronts of a launch of nwg workgroups: 4 where each gets a CU
 // of its own, so that a column is one short load batch; 2 in larger launches,
 // where the workgroups hide each other's latency and more of them at once
 // only crowd the error sinogram's atomics.  Measured (4 against 2, ms per
 // launch): 75 workgroups 0.418 / 0.704, 210 workgroups 0.310 / 0.326, 624
 // workgroups 0.660 / 0.412, 1712 workgroups 2.09 / 1.04.
+// One, where its registers hold the window, in launches of more than the five
+// workgroups of three wavefronts that a CU takes at once.  Measured (2 against
+// 1, ms per 4 equits of 256x256 columns): W = 3, 40 views per frame, 1070
+// workgroups 7.52 / 9.12, 1284 8.81 / 9.38, 1498 12.0 / 10.1; W = 3, 24 rows,
+// 1712 workgroups 15.1 / 12.4; W = 5, 896 workgroups 7.69 / 8.15, 1344 13.3 /
+// 9.51.  Wider windows stay with two: 100 views per frame, 1712 workgroups
+// 25.2 / 33.1.
 int sweep_waves(const mbir_hip_ctx* c, unsigned nwg) {
-  return sweep_pipes(c) ? 1 : (nwg <= 256 ? 4 : 2);
+  if (sweep_pipes(c) || (sweep_small(c) && nwg > 1280)) return 1;
+  return nwg <= 256 ? 4 : 2;
 }
 
 // The 8 launches per equit (2x2 tile colours x 2 frame parities) of n equits.
@@ -3374,8 +3388,7 @@ int sweep_launches(mbir_hip_ctx* c, int32_t n, int32_t first_iter, uint32_t seed
     return fail("tile slab and A windows exceed the LDS of one workgroup");
   const int nf = c->g.N_time;
   const bool timed = iter_dev == nullptr;
-  // register-light prefetch for frames of at most 64 views and 256 A values
-  const bool small = c->nvmax <= kWave && c->nvmax * c->G.W <= 4 * kWave;
+  const bool small = sweep_small(c);
   *launches = 0;
   // the equit's (colour, frame parity) sets in launch order: colour-major,
   // or with pair_parities (placement 0) (colour k, even frames) together
@@ -3447,14 +3460,16 @@ int sweep_launches(mbir_hip_ctx* c, int32_t n, int32_t first_iter, uint32_t seed
         if (timed && ev_begin(c, MBIR_K_SWEEP)) return -1;
         const int ns = sweep_waves(c, nwg);
         A.prior_sends = nwg <= 256 ? 1 : 0;
-        if (ns == 1 && small) {
-          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, true, 1>(c, A, nwg, xbytes)));
+        if (ns == 1 && !sweep_pipes(c)) {
+          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, true, 1, false>(c, A, nwg, xbytes)));
+        } else if (ns == 1 && small) {
+          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, true, 1, true>(c, A, nwg, xbytes)));
         } else if (ns == 1) {
-          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, false, 1>(c, A, nwg, xbytes)));
+          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, false, 1, true>(c, A, nwg, xbytes)));
         } else if (ns == 2) {
-          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, false, 2>(c, A, nwg, xbytes)));
+          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, false, 2, false>(c, A, nwg, xbytes)));
         } else {
-          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, false, 4>(c, A, nwg, xbytes)));
+          MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, false, 4, false>(c, A, nwg, xbytes)));
         }
         if (timed) {
           if (ev_end(c, MBIR_K_SWEEP)) return -1;
