@@ -252,10 +252,17 @@ __global__ __launch_bounds__(256) void k_swap_xy(int Ny, int Nx, int Nz, int nzc
 // 256 views of 256 bins x 8 rows, 256x256x8 voxels per frame: 0.893 -> 0.174
 // ms and 0.032 for the exchange (mode 2, FP32 atomics before: 1.604 ms); 360
 // views of 256 x 256, 256^3 voxels: 18.5 -> 7.7 ms.
+// Slices that are not a multiple of 4 read the same 16-byte loads, at any
+// float's address: 128x128x15 voxels x 8 frames of 30 views, A, e and the cost
+// 0.93 -> 0.53 ms (0.88 by the scatter).
 // The lines run along y where that is the axis of faster r; those views read
 // xt, the object with x and y exchanged (k_swap_xy), so that neighbouring
 // bins always read neighbouring voxel columns.
 constexpr int kFwdThreads = 1024;
+// four floats at any float's address: one 16-byte load on this target
+struct __attribute__((packed, aligned(4))) Float4u {
+  float x, y, z, w;
+};
 constexpr int kFwdCand = 4;
 template <int kZ, bool kWindow>
 __global__ __launch_bounds__(kFwdThreads) void k_fwdproj(
@@ -267,7 +274,10 @@ __global__ __launch_bounds__(kFwdThreads) void k_fwdproj(
     double* __restrict__ partial, double xscale) {
   extern __shared__ __align__(16) double s_acc[];  // [kFwdThreads / 2][kZ]
   __shared__ double2 s_h[kRespBins + 1];  // response and its step to the next entry; past it 0
+  // the slices [z0, z0 + kZ); the last chunk reads the last kZ, those before z0
+  // again, so that its columns are whole loads too
   const int p = blockIdx.x, z0 = blockIdx.y * kZ, nb = 1 << lognb;
+  const int zb = max(0, min(z0, G.N_z - kZ));
   const int tid = threadIdx.x, j = blockIdx.z * nb + (tid & (nb - 1)), g = tid >> lognb;
   const int ng = kFwdThreads >> lognb;
   if (tid < kRespBins) {
@@ -292,8 +302,8 @@ __global__ __launch_bounds__(kFwdThreads) void k_fwdproj(
     const double half = kRespBins * G.OffsetR * fabs(inv_a);
     const int cand = (int)(2.0 * half) + 1;
     const double centre = G.R0 + ((double)j + 0.5) * G.delta_r;
-    const float* xf = (fast_x ? x : xt) + (size_t)f * G.N_y * G.N_x * G.N_z + z0;
-    const bool vec = (G.N_z & 3) == 0 && z0 + kZ <= G.N_z;
+    const float* xf = (fast_x ? x : xt) + (size_t)f * G.N_y * G.N_x * G.N_z + zb;
+    const bool vec = G.N_z >= kZ;
     for (int u = g; u < nl; u += ng) {
       const double b = bu * u + b0;
       int i0 = (int)ceil((centre - b) * inv_a - half);
@@ -318,7 +328,7 @@ __global__ __launch_bounds__(kFwdThreads) void k_fwdproj(
           if (vec) {
 #pragma unroll
             for (int z = 0; z < kZ; z += 4) {
-              const float4 xv = *reinterpret_cast<const float4*>(xc + z);
+              const Float4u xv = *reinterpret_cast<const Float4u*>(xc + z);
               acc[z] += v * (double)(ok ? xv.x : 0.f);
               acc[z + 1] += v * (double)(ok ? xv.y : 0.f);
               acc[z + 2] += v * (double)(ok ? xv.z : 0.f);
@@ -327,7 +337,7 @@ __global__ __launch_bounds__(kFwdThreads) void k_fwdproj(
           } else {
 #pragma unroll
             for (int z = 0; z < kZ; ++z)
-              if (ok && z0 + z < G.N_z) acc[z] += v * (double)xc[z];
+              if (ok && z < G.N_z) acc[z] += v * (double)xc[z];
           }
         }
         i0 += kFwdCand;
@@ -351,9 +361,10 @@ __global__ __launch_bounds__(kFwdThreads) void k_fwdproj(
 #pragma unroll
     for (int z = 0; z < kZ; ++z) {
       const double ax = acc[z] * xscale;
+      const int zz = zb + z;
       // the slice's detector rows; the last slice also those past N_z zo
-      const int t1 = z0 + z == G.N_z - 1 ? G.N_t : (z0 + z + 1) * G.zo;
-      for (int t = (z0 + z) * G.zo; z0 + z < G.N_z && t < t1; ++t) {
+      const int t1 = zz == G.N_z - 1 ? G.N_t : (zz + 1) * G.zo;
+      for (int t = zz * G.zo; zz >= z0 && zz < G.N_z && t < t1; ++t) {
         const double axt = t < G.N_z * G.zo ? ax : 0.0;
         const size_t o = ((size_t)p * G.N_r + j) * G.N_t + t;
         const float dv = d ? d[(size_t)j * G.N_t + t] : 0.f;

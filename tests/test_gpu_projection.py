@@ -76,7 +76,8 @@ def _check(st, seed):
     (40, 34, 3, 1, 1, 1, None), (4, 520, 3, 1, 1, 1, None), (17, 130, 2, 2, 1, 1, None),
     (7, 20, 130, 2, 1, 1, None), (8, 20, 130, 2, 1, 1, 7.5), (10, 20, 70, 2, 1, 1, None),
     (13, 24, 130, 2, 1, 1, None), (16, 24, 130, 2, 2, 1, None), (20, 20, 65, 2, 1, 1, 11.0),
-    (34, 24, 130, 2, 1, 2, None)])
+    (34, 24, 130, 2, 1, 2, None), (3, 70, 4, 2, 1, 1, None), (10, 70, 65, 2, 1, 1, 31.0),
+    (17, 66, 65, 2, 1, 1, None)])
 def test_projections_match_the_system_matrix(rows, cols, views, frames, mxy, mz, rot):
     from phasecon_amd.mbir import Stage
     print(f"rows {rows}, cols {cols}, views {views} x {frames}, mult {mxy}/{mz}", flush=True)
