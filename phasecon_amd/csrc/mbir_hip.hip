@@ -257,7 +257,7 @@ __global__ __launch_bounds__(256) void k_swap_xy(int Ny, int Nx, int Nz, int nzc
 // 0.93 -> 0.53 ms (0.88 by the scatter).
 // The lines run along y where that is the axis of faster r; those views read
 // xt, the object with x and y exchanged (k_swap_xy), so that neighbouring
-// bins always read neighbouring voxel columns.
+// bins always read neighbouring voxel columns (x itself where xt is null).
 constexpr int kFwdThreads = 1024;
 // four floats at any float's address: one 16-byte load on this target
 struct __attribute__((packed, aligned(4))) Float4u {
@@ -302,7 +302,10 @@ __global__ __launch_bounds__(kFwdThreads) void k_fwdproj(
     const double half = kRespBins * G.OffsetR * fabs(inv_a);
     const int cand = (int)(2.0 * half) + 1;
     const double centre = G.R0 + ((double)j + 0.5) * G.delta_r;
-    const float* xf = (fast_x ? x : xt) + (size_t)f * G.N_y * G.N_x * G.N_z + zb;
+    // column of (line u, place i): u su + i si
+    const bool swapped = !fast_x && xt != nullptr;
+    const int su = fast_x || swapped ? ni : 1, si = fast_x || swapped ? 1 : G.N_x;
+    const float* xf = (swapped ? xt : x) + (size_t)f * G.N_y * G.N_x * G.N_z + zb;
     const bool vec = G.N_z >= kZ;
     for (int u = g; u < nl; u += ng) {
       const double b = bu * u + b0;
@@ -324,7 +327,7 @@ __global__ __launch_bounds__(kFwdThreads) void k_fwdproj(
             ok = ok && hi >= G.R0 && lo <= G.RMax && j >= jlo && j - jlo < G.W &&
                  j <= (int)floor((hi - G.R0) / G.delta_r);
           }
-          const float* xc = xf + (size_t)(ok ? u * ni + i : 0) * G.N_z;
+          const float* xc = xf + (size_t)(ok ? u * su + i * si : 0) * G.N_z;
           if (vec) {
 #pragma unroll
             for (int z = 0; z < kZ; z += 4) {
@@ -2874,13 +2877,17 @@ int run_fwdproj(mbir_hip_ctx* c, int mode, const float* x, float* out,
                         fabs(g.delta_xy - g.mult_xy * g.delta_r) <= 1e-9 * g.delta_xy &&
                         fabs(g.RMax - g.R0 - g.N_r * g.delta_r) <= 1e-9 * g.delta_xy);
   if (mode == 1 && ensure_partial(c, (size_t)q.grid.x * q.grid.y * q.grid.z)) return -1;
-  // the exchanged object, where a view reads it: in d_stage, which e and the
-  // cost leave free, so that only A x needs room for a second object
-  if (c->lines_y && mode == 2 && !c->d_xt && dev_alloc(&c->d_xt, c->nvox)) return -1;
-  float* const xt = mode == 2 ? c->d_xt : c->d_stage;
+  // the exchanged object, where a view reads it and the object has more than
+  // 64^2 columns (smaller ones lie in the caches: set-up of 33x33x7, 4 views,
+  // 149 us with the exchange, 140 without; 128x128x3, 90 views, 249 / 276): in
+  // d_stage, which e and the cost leave free, so that only A x needs room for a
+  // second object
+  const bool swap = c->lines_y && c->ncol > 64 * 64;
+  if (swap && mode == 2 && !c->d_xt && dev_alloc(&c->d_xt, c->nvox)) return -1;
+  float* const xt = !swap ? nullptr : mode == 2 ? c->d_xt : c->d_stage;
   if (ev_begin(c, mode == 1 ? MBIR_K_COST : MBIR_K_FWDPROJ)) return -1;
   const int nzc = (g.N_z + 31) / 32;
-  if (c->lines_y)
+  if (swap)
     hipLaunchKernelGGL(
         k_swap_xy, dim3((g.N_x + 15) / 16, (g.N_y + 15) / 16, std::min(65535, g.N_time * nzc)),
         dim3(256), 0, c->stream, g.N_y, g.N_x, g.N_z, nzc, g.N_time * nzc, x, xt);

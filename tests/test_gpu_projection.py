@@ -86,13 +86,15 @@ def test_projections_match_the_system_matrix(rows, cols, views, frames, mxy, mz,
     st.close()
 
 
-# every view's image lines along x, along y
+# every view's image lines along x, along y; objects that are exchanged for the
+# latter (above 64^2 columns) and that are not
+@pytest.mark.parametrize("cols", [48, 64, 65, 100])
 @pytest.mark.parametrize("lo,hi", [(-0.78, 0.78), (0.79, 2.35)])
-def test_views_of_one_axis(lo, hi):
+def test_views_of_one_axis(lo, hi, cols):
     from phasecon_amd.mbir import Stage
-    s = _scan(6, 48, 5, 2)
+    s = _scan(6, cols, 5, 2)
     s["angles"] = np.linspace(lo, hi, 10).astype(np.float32)
-    print(f"angles {lo} to {hi}", flush=True)
+    print(f"angles {lo} to {hi}, cols {cols}", flush=True)
     st = Stage(s)
     _check(st, 9)
     st.close()

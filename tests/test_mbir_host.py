@@ -18,9 +18,9 @@ def L(monkeypatch):
     return hip_stub.use(monkeypatch)
 
 
-def _scan():
+def _scan(cols=16):
     from phasecon_amd.synth import geometry_scan
-    return geometry_scan(4, 16, 6)
+    return geometry_scan(4, cols, 6)
 
 
 def _stage(**kw):
@@ -128,8 +128,8 @@ def test_grids_of_many_frames(L):
     st.backproject(np.zeros(st.shape_e, np.float32))
     st.close()
     runs = hip_stub.launches(L)
-    assert {k for k in ("k_swap_xy", "k_fwdproj", "k_backproj") if any(k in r[0] for r in runs)} \
-        == {"k_swap_xy", "k_fwdproj", "k_backproj"}
+    assert {k for k in ("k_fwdproj", "k_backproj") if any(k in r[0] for r in runs)} \
+        == {"k_fwdproj", "k_backproj"}
     for name, x, y, z, threads in runs:
         assert y <= 65535 and z <= 65535 and x * threads < 1 << 32, name
 
@@ -180,9 +180,10 @@ def test_contexts_share_the_pinned_slots(L):
 def test_the_exchanged_object_takes_no_room_of_its_own(L):
     """The error sinogram and the cost exchange x and y in the staging buffer;
     A x alone allocates for it, and nothing is exchanged where no view's lines
-    run along y."""
+    run along y, nor for an object of at most 64^2 columns."""
     from phasecon_amd.mbir import Stage
-    st = _built()
+    st = Stage(_scan(65))
+    st.build_amatrix()
     live = L.stub_live()
     st.init_error()
     assert L.stub_live() == live
@@ -190,12 +191,13 @@ def test_the_exchanged_object_takes_no_room_of_its_own(L):
     st.forward_project(np.zeros(st.shape_x, np.float32))
     assert L.stub_live() == live + 1
     st.close()
-    s = _scan()
-    s["angles"] = np.linspace(-0.7, 0.7, 6).astype(np.float32)
-    st = Stage(s)
     L.stub_clear_log()
-    st.init_error()
-    st.forward_project(np.zeros(st.shape_x, np.float32))
-    st.close()
+    flat = _scan(65)
+    flat["angles"] = np.linspace(-0.7, 0.7, 6).astype(np.float32)
+    for s in (flat, _scan(64)):
+        st = Stage(s)
+        st.init_error()
+        st.forward_project(np.zeros(st.shape_x, np.float32))
+        st.close()
     runs = [r[0] for r in hip_stub.launches(L)]
     assert any("k_fwdproj" in r for r in runs) and not any("k_swap_xy" in r for r in runs)
