@@ -2226,13 +2226,14 @@ __global__ __launch_bounds__(kWave) void k_subst(SwGeom G, float alpha, int n,
   if (act && sub == 0) out[i] = substitute(alpha, v, th1[i], th2[i], num, den);
 }
 
-// A^T v: a workgroup takes 256 columns of one frame (blockIdx.x: frame and
-// block of columns), a thread one of them and kZ slices (blockIdx.y), whose sums it keeps in registers (z_overlap rows
-// folded into z); consecutive threads take consecutive columns, which read
-// neighbouring detector rows.  The columns' A goes through LDS, `sc` view
-// slots at a time, read as each column's contiguous run: a lane reading its
-// own run slot by slot fetched every line again and again (0.935 ms), and
-// sums kept in the output array were read and written per (view, bin).
+// A^T v: a workgroup takes 256 columns of one frame (and those of every
+// 65535th after it), a thread one of them and kZ slices (blockIdx.z), whose
+// sums it keeps in registers (z_overlap rows folded into z); consecutive
+// threads take consecutive columns, which read neighbouring detector rows.  The
+// columns' A goes through LDS, `sc` view slots at a time, read as each column's
+// contiguous run: a lane reading its own run slot by slot fetched every line
+// again and again (0.935 ms), and sums kept in the output array were read and
+// written per (view, bin).
 // 256x256x8 voxels x 16 frames of 16 views: 1.75 -> 0.243 ms.
 template <int kZ>
 __global__ __launch_bounds__(256) void k_backproj(DevGeom G, int sc,
@@ -2245,58 +2246,60 @@ __global__ __launch_bounds__(256) void k_backproj(DevGeom G, int sc,
   extern __shared__ __align__(16) float smem[];
   float* s_a = smem;                                          // [sc W][257]
   int* s_f = reinterpret_cast<int*>(smem + sc * G.W * 257);   // [sc][257]
-  const int ncol = G.N_x * G.N_y, ncb = (ncol + 255) / 256, f = blockIdx.x / ncb;
-  const int c0 = (blockIdx.x - f * ncb) * 256, c = c0 + threadIdx.x, z0 = blockIdx.y * kZ;
-  const int s0 = frame_ptr[f], s1 = frame_ptr[f + 1], nc = min(256, ncol - c0);
+  const int ncol = G.N_x * G.N_y, c0 = blockIdx.x * 256, c = c0 + threadIdx.x;
+  const int z0 = blockIdx.z * kZ, nc = min(256, ncol - c0);
   const bool vec = G.zo == 1 && (G.N_t & 3) == 0 && (G.N_z & 3) == 0 && z0 + kZ <= G.N_z;
-  float acc[kZ];
+  for (int f = blockIdx.y; f < G.N_time; f += gridDim.y) {
+    const int s0 = frame_ptr[f], s1 = frame_ptr[f + 1];
+    float acc[kZ];
 #pragma unroll
-  for (int z = 0; z < kZ; ++z) acc[z] = 0.f;
-  for (int sb = s0; sb < s1; sb += sc) {
-    const int ns = min(sc, s1 - sb), na = ns * G.W;
-    __syncthreads();
-    for (int i = threadIdx.x; i < nc * na; i += 256) {
-      const int q = i / na, k = i - q * na;
-      s_a[k * 257 + q] = aval[((size_t)(c0 + q) * G.nslots + sb) * G.W + k];
-    }
-    for (int i = threadIdx.x; i < nc * ns; i += 256) {
-      const int q = i / ns, k = i - q * ns;
-      s_f[k * 257 + q] = afirst[(size_t)(c0 + q) * G.nslots + sb + k];
-    }
-    __syncthreads();
-    if (c >= ncol) continue;
-    for (int s = 0; s < ns; ++s) {
-      const int r0 = s_f[s * 257 + threadIdx.x];
-      if (r0 < 0) continue;
-      const int p = frame_views[sb + s];
-      for (int k = 0; k < G.W; ++k) {
-        const float a = s_a[(s * G.W + k) * 257 + threadIdx.x];
-        const int r = r0 + k;
-        if (a == 0.f || r >= G.N_r) continue;
-        const float* vr = v + ((size_t)p * G.N_r + r) * G.N_t + z0 * G.zo;
-        if (vec) {
+    for (int z = 0; z < kZ; ++z) acc[z] = 0.f;
+    for (int sb = s0; sb < s1; sb += sc) {
+      const int ns = min(sc, s1 - sb), na = ns * G.W;
+      __syncthreads();
+      for (int i = threadIdx.x; i < nc * na; i += 256) {
+        const int q = i / na, k = i - q * na;
+        s_a[k * 257 + q] = aval[((size_t)(c0 + q) * G.nslots + sb) * G.W + k];
+      }
+      for (int i = threadIdx.x; i < nc * ns; i += 256) {
+        const int q = i / ns, k = i - q * ns;
+        s_f[k * 257 + q] = afirst[(size_t)(c0 + q) * G.nslots + sb + k];
+      }
+      __syncthreads();
+      if (c >= ncol) continue;
+      for (int s = 0; s < ns; ++s) {
+        const int r0 = s_f[s * 257 + threadIdx.x];
+        if (r0 < 0) continue;
+        const int p = frame_views[sb + s];
+        for (int k = 0; k < G.W; ++k) {
+          const float a = s_a[(s * G.W + k) * 257 + threadIdx.x];
+          const int r = r0 + k;
+          if (a == 0.f || r >= G.N_r) continue;
+          const float* vr = v + ((size_t)p * G.N_r + r) * G.N_t + z0 * G.zo;
+          if (vec) {
 #pragma unroll
-          for (int z = 0; z < kZ; z += 4) {
-            const float4 q = *reinterpret_cast<const float4*>(vr + z);
-            acc[z] += a * q.x;
-            acc[z + 1] += a * q.y;
-            acc[z + 2] += a * q.z;
-            acc[z + 3] += a * q.w;
+            for (int z = 0; z < kZ; z += 4) {
+              const float4 q = *reinterpret_cast<const float4*>(vr + z);
+              acc[z] += a * q.x;
+              acc[z + 1] += a * q.y;
+              acc[z + 2] += a * q.z;
+              acc[z + 3] += a * q.w;
+            }
+          } else {
+#pragma unroll
+            for (int z = 0; z < kZ; ++z)
+              if (z0 + z < G.N_z)
+                for (int t = z * G.zo; t < (z + 1) * G.zo; ++t) acc[z] += a * vr[t];
           }
-        } else {
-#pragma unroll
-          for (int z = 0; z < kZ; ++z)
-            if (z0 + z < G.N_z)
-              for (int t = z * G.zo; t < (z + 1) * G.zo; ++t) acc[z] += a * vr[t];
         }
       }
     }
-  }
-  if (c >= ncol) return;
-  float* o = out + ((size_t)f * ncol + c) * G.N_z + z0;
+    if (c >= ncol) continue;
+    float* o = out + ((size_t)f * ncol + c) * G.N_z + z0;
 #pragma unroll
-  for (int z = 0; z < kZ; ++z)
-    if (z0 + z < G.N_z) o[z] = acc[z];
+    for (int z = 0; z < kZ; ++z)
+      if (z0 + z < G.N_z) o[z] = acc[z];
+  }
 }
 
 // Normalised back-projection: per voxel sum(w a (y - d)) / sum(w a (A m))
@@ -2918,7 +2921,7 @@ void launch_sweep(mbir_hip_ctx* c, const SweepArgs& A, unsigned nwg, size_t lds)
 // chunk of slices reads the stored A again).
 void launch_backproj(mbir_hip_ctx* c, const float* v, float* out) {
   const int kz = c->g.N_z <= 8 ? 8 : 32;
-  const dim3 grid((unsigned)((c->ncol + 255) / 256) * (unsigned)c->g.N_time,
+  const dim3 grid((unsigned)((c->ncol + 255) / 256), (unsigned)std::min(65535, c->g.N_time),
                   (unsigned)((c->g.N_z + kz - 1) / kz));
   // 32 KiB of A at a time (W = 33: one slot, 35 KiB)
   const int sc = std::max(1, 32 / (1 + c->G.W));
