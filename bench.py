@@ -101,9 +101,9 @@ REL_TOL = 1e-5
 # line carries this figure with its source.
 # Keyed by (workload, tile, FP16 A, paired parities): a paired launch holds
 # two (colour, frame parity) sets.
-MEASURED_TRAFFIC = {("ch4d", 8, False, False): 145609.5 * 1024 * 2.0 + 120815.1 * 1024 * 1.0,
-                    ("ch4d", 8, False, True): 301410.4 * 1024 * 2.0 + 241630.7 * 1024 * 1.0,
-                    ("ch4d", 12, False, True): 310021.1 * 1024 * 2.0 + 241499.1 * 1024 * 1.0}
+MEASURED_TRAFFIC = {("ch4d", 8, False, False): 149713.2 * 1024 * 2.0 + 120815.0 * 1024 * 1.0,
+                    ("ch4d", 8, False, True): 300595.5 * 1024 * 2.0 + 241630.1 * 1024 * 1.0,
+                    ("ch4d", 12, False, True): 310392.9 * 1024 * 2.0 + 241499.1 * 1024 * 1.0}
 TRAFFIC_SOURCE = "profiles/k_sweep_ch4d_counters.md (rocprofv3 --pmc FETCH_SIZE, WRITE_SIZE)"
 
 
