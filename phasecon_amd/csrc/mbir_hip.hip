@@ -810,11 +810,15 @@ struct Lanes {
 // row's sums lands in row1 / row2.  Each lane issues the e/w loads of a batch
 // of its slots back to back, then accumulates; entries with a = 0 load the
 // sinogram's first element and are not used, so that no branch splits the
-// batch.
-template <int kW>
+// batch.  kBusy: a launch that fills the chip by one wavefront per workgroup;
+// from W = 5 on its batches are smaller, for 5 wavefronts per SIMD instead of 3
+// (93 registers, not 137; 256x256x6 x 8 frames of 30 views, W = 5: 9.49 -> 7.43
+// ms per 2 equits; W = 9 9.78 -> 9.41; W = 3 would lose, 11.0 -> 11.4).
+template <int kW, bool kBusy = false>
 __device__ __forceinline__ void col_thetas(const SwGeom& G, const ColumnArgs& A, const Win& win,
                                            int nv, int wv, int nw, float* row1, float* row2) {
-  constexpr int SB = kW <= 5 ? 4 : (kW <= 9 ? 2 : 1);  // slots per load batch
+  // slots per load batch
+  constexpr int SB = kBusy ? (kW <= 3 ? 4 : kW <= 5 ? 2 : 1) : kW <= 5 ? 4 : (kW <= 9 ? 2 : 1);
   const Lanes L(G.N_t);
   const int step = nw * L.groups;
   const float T2 = G.huber_T * G.huber_T, Thd = G.huber_T * G.huber_delta;
@@ -1490,7 +1494,8 @@ k_sweep(SwGeom G, SweepArgs A) {
         awin_fetch<kW, kSmall, kHalf, kNS>(G, A.col, cn, s0, nv, tid, pre);
         tn_fetch(G, A.x, f, cn, vol, tid, pre);
       }
-      col_thetas<kW>(G, A.col, wcur, nv, wv, kNS, s_row1 + wv * kNTMax, s_row2 + wv * kNTMax);
+      col_thetas<kW, kNS == 1>(G, A.col, wcur, nv, wv, kNS, s_row1 + wv * kNTMax,
+                               s_row2 + wv * kNTMax);
       __syncthreads();
       // phase 2: store the prefetch (it landed with the theta loads) and
       // retire every load explicitly (a free wait here) so that the

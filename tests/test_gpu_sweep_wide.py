@@ -100,3 +100,40 @@ def test_wide_sweep_in_large_launches(rows, views):
     # six equits of about 200 atomic additions per entry, each rounded to 2^-24
     assert d < 2e-5
     assert costs[-1] < 0.5 * costs[0]
+
+
+# 16 tiles per colour x 85 frames of a parity: one wavefront on the sinogram
+# side, load batches of W = 5 and W = 9
+@pytest.mark.parametrize("rows,views,mxy", [(6, 9, 2), (3, 21, 2), (6, 7, 4)])
+def test_busy_sweep_of_wide_bins(rows, views, mxy):
+    from phasecon_amd.mbir import Stage
+    from phasecon_amd.synth import make_scan
+    scan = make_scan("tall3d", seed=4, rows=rows, cols=32 * mxy, views=views * 170, frames=170)
+    print(f"rows {rows}, views {views} x 170, mult_xy {mxy}", flush=True)
+    st = Stage(scan, mult_xy=mxy, tile=4, alpha=1.0)
+    st.build_amatrix()
+    st.init_error()
+    costs = [st.cost()[0]]
+    for it in range(1, 7):
+        st.icd(1, it)
+        costs.append(st.cost()[0])
+    kept = st.get_error().astype(np.float64)
+    x, st2 = st.get_object(), Stage(scan, mult_xy=mxy, tile=16, alpha=1.0)
+    st.init_error()
+    fresh = st.get_error().astype(np.float64)
+    st.close()
+    # the same equits with few, larger tiles, two wavefronts: near the same object
+    st2.build_amatrix()
+    st2.init_error()
+    for it in range(1, 7):
+        st2.icd(1, it)
+    c2 = st2.cost()[0]
+    st2.close()
+    d = np.abs(kept - fresh).max() / np.abs(st.y).max()
+    print(f"kept e off by {d:.3g}, costs {costs[0]:.6g} -> {costs[-1]:.6g}, tile 16 {c2:.6g}",
+          flush=True)
+    # as above; after six equits neither schedule is at the optimum, but both
+    # costs are a few per cent of the first, and so is what they differ by
+    assert d < 2e-5
+    assert np.isfinite(x).all() and costs[-1] < 0.1 * costs[0]
+    assert abs(costs[-1] - c2) < 0.02 * costs[0]
