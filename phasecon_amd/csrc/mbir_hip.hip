@@ -2912,6 +2912,59 @@ int run_fwdproj(mbir_hip_ctx* c, int mode, const float* x, float* out,
   return ev_end(c, mode == 1 ? MBIR_K_COST : MBIR_K_FWDPROJ);
 }
 
+// The pipelined sweep (one sinogram wavefront) runs where the largest frame's
+// window is one load batch of that wavefront: N_t a power of two up to 64 and
+// nvmax <= SB (64 / N_t) slots, SB = 2 up to W = 5, else 1.
+bool sweep_pipes(const mbir_hip_ctx* c) {
+  const int nt = c->g.N_t;
+  return nt <= kWave && (nt & (nt - 1)) == 0 &&
+         c->nvmax <= (c->G.W <= 5 ? 2 : 1) * (kWave / nt);
+}
+
+// Frames whose window one wavefront stages in 1 + 4 registers per lane.
+bool sweep_small(const mbir_hip_ctx* c) {
+  return c->nvmax <= kWave && c->nvmax * c->G.W <= 4 * kWave;
+}
+
+// Workgroups of a kernel that the chip's 256 CUs hold at once.
+template <typename K>
+unsigned chip_holds(K kernel, int threads, size_t lds) {
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, threads, lds) != hipSuccess || n < 1)
+    n = 1;
+  return 256u * (unsigned)n;
+}
+
+// Sinogram wavefronts of a launch of nwg workgroups with `lds` bytes: 4 where
+// each gets a CU of its own, so that a column is one short load batch; 2 in
+// larger launches, where the workgroups hide each other's latency and more of
+// them at once only crowd the error sinogram's atomics.  Measured (4 against
+// 2, ms per launch): 75 workgroups 0.418 / 0.704, 210 workgroups 0.310 /
+// 0.326, 624 workgroups 0.660 / 0.412, 1712 workgroups 2.09 / 1.04.
+// One, where its registers hold the window, in launches that it brings through
+// the chip in so many fewer rounds that its longer round pays: the chip holds 8
+// to 11 workgroups of two wavefronts per CU, 4 or 5 of three, whose round takes
+// 0.82 of one wavefront's at W = 3, about 0.6 above (a last round of less than
+// 2 % is not counted).  Measured (2 against 1, ms for 2 or 4 equits, rounds in
+// brackets): W = 3, 1070 workgroups 7.52 / 9.12 (1 / 1), 1284 8.81 / 9.38 (1 /
+// 1), 1498 12.0 / 10.1 (2 / 1), 1712 15.1 / 12.4 (2 / 1); W = 5, 896 7.69 / 8.15
+// (1 / 1), 1064 12.7 / 9.67 (2 / 1), 1712 8.54 / 7.43 (2 / 1); W = 9, 2240 14.6 /
+// 13.5 (2 / 1); W = 17, 2240 5.08 / 6.23 (2 / 2), 3584 7.54 / 7.85 (3 / 2).
+// Wider windows stay with two: W = 3, 100 views per frame, 1712 workgroups 25.2 /
+// 33.1.
+template <int kW>
+int sweep_waves(const mbir_hip_ctx* c, unsigned nwg, size_t lds) {
+  if (sweep_pipes(c)) return 1;
+  if (nwg <= 256) return 4;
+  if (!sweep_small(c)) return 2;
+  const unsigned one = c->afp16 ? chip_holds(k_sweep<kW, true, true, 1, false>, 2 * kWave, lds)
+                                : chip_holds(k_sweep<kW, true, false, 1, false>, 2 * kWave, lds);
+  const unsigned two = c->afp16 ? chip_holds(k_sweep<kW, false, true, 2, false>, 3 * kWave, lds)
+                                : chip_holds(k_sweep<kW, false, false, 2, false>, 3 * kWave, lds);
+  const auto rounds = [nwg](unsigned holds) { return (nwg + holds - 1 - holds / 50) / holds; };
+  return rounds(one) * 100 < rounds(two) * (kW == 3 ? 82 : 62) ? 1 : 2;
+}
+
 template <int kW, bool kSmall, int kNS, bool kPipe>
 void launch_sweep(mbir_hip_ctx* c, const SweepArgs& A, unsigned nwg, size_t lds) {
   if (c->afp16)
@@ -3341,38 +3394,6 @@ int mbir_sweep_fits(const mbir_hip_ctx* c) {
   return 0;
 }
 
-// The pipelined sweep (one sinogram wavefront) runs where the largest frame's
-// window is one load batch of that wavefront: N_t a power of two up to 64 and
-// nvmax <= SB (64 / N_t) slots, SB = 2 up to W = 5, else 1.
-bool sweep_pipes(const mbir_hip_ctx* c) {
-  const int nt = c->g.N_t;
-  return nt <= kWave && (nt & (nt - 1)) == 0 &&
-         c->nvmax <= (c->G.W <= 5 ? 2 : 1) * (kWave / nt);
-}
-
-// Frames whose window one wavefront stages in 1 + 4 registers per lane.
-bool sweep_small(const mbir_hip_ctx* c) {
-  return c->nvmax <= kWave && c->nvmax * c->G.W <= 4 * kWave;
-}
-
-// Sinogram wavefronts of a launch of nwg workgroups: 4 where each gets a CU
-// of its own, so that a column is one short load batch; 2 in larger launches,
-// where the workgroups hide each other's latency and more of them at once
-// only crowd the error sinogram's atomics.  Measured (4 against 2, ms per
-// launch): 75 workgroups 0.418 / 0.704, 210 workgroups 0.310 / 0.326, 624
-// workgroups 0.660 / 0.412, 1712 workgroups 2.09 / 1.04.
-// One, where its registers hold the window, in launches of more than the five
-// workgroups of three wavefronts that a CU takes at once.  Measured (2 against
-// 1, ms per 4 equits of 256x256 columns): W = 3, 40 views per frame, 1070
-// workgroups 7.52 / 9.12, 1284 8.81 / 9.38, 1498 12.0 / 10.1; W = 3, 24 rows,
-// 1712 workgroups 15.1 / 12.4; W = 5, 896 workgroups 7.69 / 8.15, 1344 13.3 /
-// 9.51.  Wider windows stay with two: 100 views per frame, 1712 workgroups
-// 25.2 / 33.1.
-int sweep_waves(const mbir_hip_ctx* c, unsigned nwg) {
-  if (sweep_pipes(c) || (sweep_small(c) && nwg > 1280)) return 1;
-  return nwg <= 256 ? 4 : 2;
-}
-
 // The 8 launches per equit (2x2 tile colours x 2 frame parities) of n equits.
 // iter_dev null: iterations first_iter .. first_iter + n - 1, each launch
 // timed; otherwise the iteration is *iter_dev + it (graph capture: no event
@@ -3484,7 +3505,8 @@ int sweep_launches(mbir_hip_ctx* c, int32_t n, int32_t first_iter, uint32_t seed
           nwg += (unsigned)(set_ntl(b) * set_frames(b));
         }
         if (timed && ev_begin(c, MBIR_K_SWEEP)) return -1;
-        const int ns = sweep_waves(c, nwg);
+        int ns = 0;
+        MBIR_DISPATCH_W(c->G.W, ns = sweep_waves<kW>(c, nwg, xbytes));
         A.prior_sends = nwg <= 256 ? 1 : 0;
         if (ns == 1 && !sweep_pipes(c)) {
           MBIR_DISPATCH_W(c->G.W, (launch_sweep<kW, true, 1, false>(c, A, nwg, xbytes)));

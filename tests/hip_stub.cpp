@@ -147,6 +147,10 @@ hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) {
   *v = 160 * 1024;  // the only one asked for: LDS per workgroup
   return hipSuccess;
 }
+hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void*, int threads, size_t) {
+  *n = 2048 / threads;
+  return hipSuccess;
+}
 hipError_t hipGetSymbolAddress(void** p, const void* s) {
   *p = const_cast<void*>(s);
   return hipSuccess;
